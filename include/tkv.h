@@ -294,6 +294,16 @@ int tkv_unpack_dequant(const uint8_t *packed, const uint16_t *scale, const uint1
                        int32_t path, uint8_t *codes_out, float *values_out,
                        tkv_stream_t stream);
 
+/* Rows of a quantized cache back to values or codes: out_type 0 fp32, 1 fp16,
+ * 2 bf16 (fp32 code * scale + zero, rounded once), 3 uint8 codes (scale and
+ * zero unused).  out is (rows, D), 16-byte aligned (codes: 8), packed 8-byte
+ * aligned.  The same values as tkv_unpack_dequant, written by a kernel laid
+ * out for whole caches.  As dequantize_groupwise / unpack_codes
+ * (quantize.py:239-246, :172-183). */
+int tkv_dequantize(const uint8_t *packed, const uint16_t *scale, const uint16_t *zero,
+                   int64_t rows, int32_t D, int32_t nbits, int32_t group_size, int32_t out_type,
+                   void *out, tkv_stream_t stream);
+
 typedef struct tkv_device_info_t {
   int32_t device;
   int32_t compute_units;

@@ -110,6 +110,7 @@ SIGNATURES = {
                                   _P, _P, _P, _P, _P, _P, _P], ctypes.c_int),
     "tkv_pack_codes": ([_P, _I64, _I32, _I32, _P, _P], ctypes.c_int),
     "tkv_unpack_dequant": ([_P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P, _P, _P], ctypes.c_int),
+    "tkv_dequantize": ([_P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P, _P], ctypes.c_int),
     "tkv_device_info": ([ctypes.POINTER(DeviceInfo)], ctypes.c_int),
     "tkv_status_string": ([ctypes.c_int], ctypes.c_char_p),
     "tkv_abi_version": ([], ctypes.c_int),

@@ -38,7 +38,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libtkv_hip.so")
-SOURCES = ["decode_attention.hip", "quant_pack.hip", "runtime.hip"] + [
+SOURCES = ["decode_attention.hip", "quant_pack.hip", "dequant.hip", "runtime.hip"] + [
     f"quant_split_{bits}{hc}.hip" for bits in ("k4v4", "k2v2", "k4v2", "k2v4") for hc in ("", "_h4", "_h8")]
 ARCH = "gfx950"
 
