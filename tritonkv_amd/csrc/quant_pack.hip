@@ -31,6 +31,13 @@ struct PageMap {
   int stride, page_size, num_pages;
 };
 
+// Rows to quantize: value d of token t of (b, kv head) is element
+// b * sb + kv * sh + t * st + d of x.
+struct TokenSource {
+  const void* x;
+  int64_t sb, sh, st;
+};
+
 // One wave per cache row (token x kv head), quantized by quantize_row: lane j
 // owns packed byte j of the row.  Used when the input or the codes are not
 // aligned for the wide kernel below.
@@ -68,125 +75,162 @@ quantize_pack_kernel(const void* __restrict__ x, int64_t row0, int64_t rows, int
   }
 }
 
-// Bulk form of the same quantization (the same arithmetic, so the same bits):
-// lane (slot r = l / LPR, column c = l % LPR) owns the E = 8 packed bytes
-// [8c, 8c + 8) of its row, i.e. the 8P codes of dims 8c + e + p*DP.  It reads
-// P runs of 8 consecutive values (16-byte loads) and writes its 8 bytes in one
-// store.  Group min/max fold the lane's own 8 values, then run over the GS/8
-// lanes of the group (or, when a group spans GS/DP slices, over the row's LPR
-// lanes) by DPP.  A wave covers 64/LPR rows per step; with BULK it takes
-// STEPS steps of rows, all their loads issued before any arithmetic.
-// Requires x 16-byte and packed 8-byte aligned, rows < 2^31.
+// The same quantization spread over lanes eight bytes at a time (the same
+// arithmetic, so the same bits).  A lane (slot r = l / LPR, column c = l % LPR)
+// owns the E = 8 packed bytes [8c, 8c + 8) of its row, i.e. the 8P codes of
+// dims 8c + e + p*DP: P runs of 8 consecutive values (16-byte loads) in, one
+// 8-byte store of codes out.
+template <int D, int NB, int GS, bool F32>
+struct WideRow {
+  static constexpr int P = 8 / NB, DP = D / P, NG = D / GS, QMAX = (1 << NB) - 1, E = 8;
+  static constexpr int LPR = DP / E, RPS = 64 / LPR;  // lanes per row, rows per wave and step
+  static constexpr int NV = F32 ? 2 : 1;              // 16-byte loads per run of E values
+  static_assert(DP % E == 0 && LPR >= 2 && LPR <= 16, "row shape");
+  static_assert(GS > DP ? GS % DP == 0 : GS % E == 0, "group shape");
+
+  // Whether this lane holds the first byte of a group of slice p, and which group.
+  __device__ static bool first_byte(int c, int p) {
+    if constexpr (GS <= DP) return (c * E) % GS == 0;
+    else return c == 0 && p % (GS / DP) == 0;
+  }
+  __device__ static constexpr int group_of(int c, int p) { return (p * DP + c * E) / GS; }
+
+  __device__ static void load(const void* x, int64_t off, int c, u4 (&raw)[P][NV]) {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        // read once: non-temporal (35.2 -> 31.5 us for the 4-bit rows below)
+        const int64_t e = off + p * DP + c * E;
+        const u4* v = F32 ? reinterpret_cast<const u4*>(static_cast<const float*>(x) + e)
+                          : reinterpret_cast<const u4*>(static_cast<const _Float16*>(x) + e);
+        raw[p][k] = __builtin_nontemporal_load(v + k);
+      }
+  }
+
+  // Value e of a run.  fp32: whole-vector casts (this compiler folds a min/max
+  // over floats cast one by one from an integer vector's elements to the first).
+  __device__ static float value(const u4 (&raw)[NV], int e) {
+    if constexpr (F32) return __builtin_bit_cast(f4, raw[e / 4])[e % 4];
+    else return (float)__builtin_bit_cast(h8, raw[0])[e];
+  }
+
+  // The lane's 8 code bytes, and each slice's fp16 scale (low half) and zero.
+  __device__ static void quantize(const u4 (&raw)[P][NV], u2& codes, uint32_t (&sz)[P]) {
+    float mn[P], mx[P];
+    if constexpr (F32) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        mn[p] = mx[p] = value(raw[p], 0);
+#pragma unroll
+        for (int e = 1; e < E; ++e) {
+          mn[p] = nan_min(mn[p], value(raw[p], e));
+          mx[p] = nan_max(mx[p], value(raw[p], e));
+        }
+      }
+      if constexpr (GS <= DP) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) minmax_lanes<GS / E>(mn[p], mx[p]);
+      } else {
+        constexpr int SPG = GS / DP;
+#pragma unroll
+        for (int p = 0; p < P; p += SPG) {
+#pragma unroll
+          for (int e = 1; e < SPG; ++e) {
+            mn[p] = nan_min(mn[p], mn[p + e]);
+            mx[p] = nan_max(mx[p], mx[p + e]);
+          }
+          minmax_lanes<LPR>(mn[p], mx[p]);
+#pragma unroll
+          for (int e = 1; e < SPG; ++e) mn[p + e] = mn[p], mx[p + e] = mx[p];
+        }
+      }
+    } else {
+      // fp16 values are their own min and max: packed v_pk_minimum3 / maximum3
+      // fold the run, then (min, -max) travels as one fp16 pair.
+      h2 mm[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) mm[p] = run_minmax(raw[p][0]);
+      if constexpr (GS <= DP) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) mm[p] = pair_min_lanes<GS / E>(mm[p]);
+      } else {
+        constexpr int SPG = GS / DP;
+#pragma unroll
+        for (int p = 0; p < P; p += SPG) {
+#pragma unroll
+          for (int e = 1; e < SPG; ++e) mm[p] = __builtin_elementwise_minimum(mm[p], mm[p + e]);
+          mm[p] = pair_min_lanes<LPR>(mm[p]);
+#pragma unroll
+          for (int e = 1; e < SPG; ++e) mm[p + e] = mm[p];
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        mn[p] = (float)mm[p][0];
+        mx[p] = -(float)mm[p][1];
+      }
+    }
+    float sf[P], zf[P], special = 0.0f;
+    uint32_t w[2] = {code_bias<P, NB>(), code_bias<P, NB>()};
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const GroupScale g = group_scale<QMAX>(mn[p], mx[p]);
+      sz[p] = g.bits;
+      sf[p] = g.s;
+      zf[p] = g.z;
+      const float rs = __builtin_amdgcn_rcpf(g.s);
+      special += group_special(g.s, g.z, rs);
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        w[e / 4] += code_term<QMAX>(value_less(raw[p], e, g.z), g.s, rs) << (8 * (e % 4) + p * NB);
+    }
+    if (__builtin_expect(special != 0.0f, 0)) {  // NaN: redo the lane's codes by division
+      w[0] = w[1] = 0;
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          w[e / 4] |= code_by_division<QMAX>(value(raw[p], e) - zf[p], sf[p]) << (8 * (e % 4) + p * NB);
+    }
+    codes = u2{w[0], w[1]};
+  }
+
+ private:
+  // Value e of a run less z; fp16 as one v_fma_mix (the opaque 1.0 keeps the
+  // conversion inside the multiply-add: one rounding, that of the difference).
+  __device__ static float value_less(const u4 (&raw)[NV], int e, float z) {
+    if constexpr (F32) return value(raw, e) - z;
+    else return half_less(raw[0][e / 2], e & 1, z);
+  }
+};
+
+// A few rows, and paged caches: each wave finds its rows' batch row, head and
+// destination by division.  BULK takes several steps of rows, all their loads
+// issued before any arithmetic.  Requires x 16-byte and packed 8-byte aligned,
+// rows < 2^31.
 template <int D, int NB, int GS, bool F32, bool BULK>
 __global__ void __launch_bounds__(256)
 quantize_pack_wide_kernel(const void* __restrict__ x, int rows, int HKV, int N,
                           const int32_t* __restrict__ positions, int S_cap, PageMap pm,
                           uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
                           uint16_t* __restrict__ zero) {
-  constexpr int P = 8 / NB, DP = D / P, NG = D / GS, QMAX = (1 << NB) - 1, E = 8;
-  constexpr int LPR = DP / E, RPS = 64 / LPR;
-  constexpr int NV = F32 ? 2 : 1;  // 16-byte loads per run of E values
-  constexpr int STEPS = BULK ? (8 / (P * NV) > 0 ? 8 / (P * NV) : 1) : 1;  // ~128 B per lane
-  static_assert(DP % E == 0 && LPR >= 2 && LPR <= 16, "row shape");
-  static_assert(GS > DP ? GS % DP == 0 : GS % E == 0, "group shape");
+  using W = WideRow<D, NB, GS, F32>;
+  constexpr int P = W::P, DP = W::DP, NG = W::NG, RPS = W::RPS;
+  constexpr int STEPS = BULK ? (8 / (P * W::NV) > 0 ? 8 / (P * W::NV) : 1) : 1;  // ~128 B per lane
 
-  const int lane = threadIdx.x & 63, slot = lane / LPR, c = lane % LPR;
+  const int lane = threadIdx.x & 63, slot = lane / W::LPR, c = lane % W::LPR;
   const int first = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * STEPS * RPS;
-  u4 raw[STEPS][P][NV];
+  u4 raw[STEPS][P][W::NV];
 #pragma unroll
-  for (int s = 0; s < STEPS; ++s) {
-    int rr = first + s * RPS + slot;
-    if (rr >= rows) rr = rows - 1;
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int64_t off = (int64_t)rr * D + p * DP + c * E;  // elements
-#pragma unroll
-      for (int k = 0; k < NV; ++k)
-        raw[s][p][k] = F32 ? reinterpret_cast<const u4*>(static_cast<const float*>(x) + off)[k]
-                           : reinterpret_cast<const u4*>(static_cast<const _Float16*>(x) + off)[k];
-    }
-  }
+  for (int s = 0; s < STEPS; ++s)
+    W::load(x, (int64_t)min(first + s * RPS + slot, rows - 1) * D, c, raw[s]);
 #pragma unroll
   for (int s = 0; s < STEPS; ++s) {
     const int rr = first + s * RPS + slot;
-    float v[P][E], mn[P], mx[P];
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      if constexpr (F32) {
-        // Whole-vector casts: this compiler folds a min/max over floats cast
-        // one by one from the elements of an integer vector to the first one.
-        const f4 lo = __builtin_bit_cast(f4, raw[s][p][0]), hi = __builtin_bit_cast(f4, raw[s][p][1]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[p][e] = lo[e], v[p][e + 4] = hi[e];
-      } else {
-        const h8 h = __builtin_bit_cast(h8, raw[s][p][0]);
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[p][e] = (float)h[e];
-      }
-      mn[p] = mx[p] = v[p][0];
-#pragma unroll
-      for (int e = 1; e < E; ++e) {
-        mn[p] = nan_min(mn[p], v[p][e]);
-        mx[p] = nan_max(mx[p], v[p][e]);
-      }
-    }
-    if constexpr (GS <= DP) {
-#pragma unroll
-      for (int p = 0; p < P; ++p) minmax_lanes<GS / E>(mn[p], mx[p]);
-    } else {
-      constexpr int SPG = GS / DP;
-#pragma unroll
-      for (int p = 0; p < P; p += SPG) {
-#pragma unroll
-        for (int e = 1; e < SPG; ++e) {
-          mn[p] = nan_min(mn[p], mn[p + e]);
-          mx[p] = nan_max(mx[p], mx[p + e]);
-        }
-        minmax_lanes<LPR>(mn[p], mx[p]);
-#pragma unroll
-        for (int e = 1; e < SPG; ++e) {
-          mn[p + e] = mn[p];
-          mx[p + e] = mx[p];
-        }
-      }
-    }
-    float sf[P], zf[P], q[P][E];
-    uint16_t s16b[P], z16b[P];
-    bool unsure = false;
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      float sc = (mx[p] - mn[p]) / (float)QMAX;
-      if (!(sc > 0.0f)) sc = 1.0f;
-      const _Float16 s16 = (_Float16)sc;
-      const _Float16 z16 = (_Float16)mn[p];
-      sf[p] = (float)s16;
-      zf[p] = (float)z16;
-      s16b[p] = __builtin_bit_cast(uint16_t, s16);
-      z16b[p] = zero_bits(mn[p]);
-      const float rs = __builtin_amdgcn_rcpf(sf[p]);
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const float y = (v[p][e] - zf[p]) * rs;
-        q[p][e] = rintf(y);
-        unsure |= quotient_unsure(y, q[p][e]);
-      }
-    }
-    if (__builtin_expect(unsure, 0)) {  // rare: redo the lane's codes by division
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-#pragma unroll
-        for (int e = 0; e < E; ++e) q[p][e] = rintf((v[p][e] - zf[p]) / sf[p]);
-    }
-    uint32_t w[2] = {0, 0};
-#pragma unroll
-    for (int p = 0; p < P; ++p)
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        float c = q[p][e];
-        if (c != c) c = 0.0f;
-        c = fminf(fmaxf(c, 0.0f), (float)QMAX);
-        w[e / 4] |= (uint32_t)c << (8 * (e % 4) + p * NB);
-      }
+    u2 codes;
+    uint32_t sz[P];
+    W::quantize(raw[s], codes, sz);
     if (rr >= rows) continue;  // after the cross-lane steps, which need every lane
     const int bh = rr / N, t = rr - bh * N;
     const int b = bh / HKV, kv = bh - b * HKV;
@@ -199,19 +243,94 @@ quantize_pack_wide_kernel(const void* __restrict__ x, int rows, int HKV, int N,
       dst_row = ((int64_t)e * HKV + kv) * pm.page_size + dst_t % pm.page_size;
     }
     if (!in_range) continue;
-    *reinterpret_cast<u2*>(packed + dst_row * DP + c * E) = u2{w[0], w[1]};
+    *reinterpret_cast<u2*>(packed + dst_row * DP + c * W::E) = codes;
     // Group g's scale and zero are written by the lane holding its first byte.
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      bool first_byte;
-      if constexpr (GS <= DP) first_byte = (c * E) % GS == 0;
-      else first_byte = c == 0 && p % (GS / DP) == 0;
-      if (first_byte) {
-        const int g = (p * DP + c * E) / GS;
-        scale[dst_row * NG + g] = s16b[p];
-        zero[dst_row * NG + g] = z16b[p];
+    for (int p = 0; p < P; ++p)
+      if (W::first_byte(c, p)) {
+        scale[dst_row * NG + W::group_of(c, p)] = (uint16_t)sz[p];
+        zero[dst_row * NG + W::group_of(c, p)] = (uint16_t)(sz[p] >> 16);
+      }
+  }
+}
+
+// A prompt's rows (many tokens per head) into a contiguous cache: HBM-bound
+// with VALU close behind, so a workgroup's tokens all belong to one (b, kv
+// head), whose addresses are scalar, and the metadata of a wave's rows meets
+// in LDS and leaves as whole dwords (64 lanes store 256 consecutive bytes,
+// where each group's first lane used to store its own 2 bytes).  524288 rows of
+// D = 128 fp16, groups of 32: 4-bit 53 -> 31.5 us (5.6 TB/s), 2-bit 54 -> 30.4
+// us (5.2 TB/s); the gain is VALU: 1.1k -> 0.8k instructions per 32 rows from
+// the exact quotient that needs no fallback for ties, packed fp16 min/max and
+// no integer divisions.
+// Workgroup x takes tile x / HKV of head x % HKV when the source is
+// token-major (tile % tiles of head x / tiles otherwise), so that workgroups
+// running together read neighbouring memory; y is the batch row.
+// Requires x 16-byte, its strides 16-byte multiples, packed 8-byte and
+// scale / zero 4-byte aligned.
+template <int D, int NB, int GS, bool F32, int STEPS>
+__global__ void __launch_bounds__(256)
+quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
+                       const int32_t* __restrict__ positions, int S_cap,
+                       uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
+                       uint16_t* __restrict__ zero) {
+  using W = WideRow<D, NB, GS, F32>;
+  constexpr int P = W::P, DP = W::DP, NG = W::NG, RPS = W::RPS, ROWS = STEPS * RPS;
+  __shared__ __attribute__((aligned(16))) uint32_t meta_lds[4][ROWS * NG];
+
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int slot = lane / W::LPR, c = lane % W::LPR;
+  const bool heads_first = src.st != D;
+  const int q = (int)blockIdx.x / (heads_first ? HKV : tiles);
+  const int m = (int)blockIdx.x - q * (heads_first ? HKV : tiles);
+  const int kv = heads_first ? m : q, tile = heads_first ? q : m, b = blockIdx.y;
+  const int t0 = (tile * 4 + w) * ROWS;
+  if (t0 >= N) return;  // whole wave
+  const int64_t base = b * src.sb + kv * src.sh + t0 * src.st;
+  u4 raw[STEPS][P][W::NV];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s)
+    W::load(src.x, base + (int64_t)min(s * RPS + slot, N - 1 - t0) * src.st, c, raw[s]);
+
+  // Token t0 + i of the wave goes to row dst0 + i of the (b, kv head) block; rows
+  // i in [lo, hi) exist and fit the capacity.
+  const int64_t dst0 = (int64_t)(positions ? positions[b] : 0) + t0;
+  const int64_t left = max((int64_t)S_cap - dst0, (int64_t)0);
+  const int lo = (int)min(max(-dst0, (int64_t)0), (int64_t)ROWS);
+  const int hi = (int)min((int64_t)min(ROWS, N - t0), left);
+  const int64_t row0 = ((int64_t)b * HKV + kv) * S_cap + dst0;
+  uint32_t* const meta = meta_lds[w];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    u2 codes;
+    uint32_t sz[P];
+    W::quantize(raw[s], codes, sz);
+    const int i = s * RPS + slot;
+    if (i >= lo && i < hi) *reinterpret_cast<u2*>(packed + (row0 + i) * DP + c * W::E) = codes;
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+      if (W::first_byte(c, p)) meta[i * NG + W::group_of(c, p)] = sz[p];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if constexpr (NG >= 2) {
+#pragma unroll
+    for (int k = lane; k < ROWS * NG / 2; k += 64) {  // dword k: groups 2k, 2k + 1 of the wave's rows
+      const int i = 2 * k / NG;
+      const u2 two = *reinterpret_cast<const u2*>(meta + 2 * k);
+      if (i >= lo && i < hi) {
+        reinterpret_cast<uint32_t*>(scale + row0 * NG)[k] = perm(two[1], two[0], 0x05040100u);
+        reinterpret_cast<uint32_t*>(zero + row0 * NG)[k] = perm(two[1], two[0], 0x07060302u);
       }
     }
+  } else {
+#pragma unroll
+    for (int i = lane; i < ROWS; i += 64)
+      if (i >= lo && i < hi) {
+        scale[row0 + i] = (uint16_t)meta[i];
+        zero[row0 + i] = (uint16_t)(meta[i] >> 16);
+      }
   }
 }
 
@@ -488,23 +607,42 @@ unpack_v_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__
   }
 }
 
+// Tokens per head from which a workgroup takes tokens of one head only
+// (quantize_tokens_kernel).  Below it most of a workgroup's rows would be
+// empty, and the rows of all heads are run together (quantize_pack_wide_kernel).
+constexpr int kTokensMinN = 32;
+// Rows from which a wave takes several steps of rows: fewer rows run one step
+// per wave, at most eight waves for each of the chip's 1024 SIMDs.
+constexpr int64_t kBulkRows = 65536;
+
 template <int D, int NB, int GS>
-static void launch_quantize(const void* x, bool f32, int64_t rows, int HKV, int N,
+static void launch_quantize(const TokenSource& src, bool f32, int B, int HKV, int N,
                             const int32_t* pos, int S_cap, PageMap pm, uint8_t* pk, uint16_t* sc,
                             uint16_t* zr, hipStream_t st) {
-  // The wide kernel needs 16-byte aligned input and 8-byte aligned codes;
-  // otherwise one wave per row.  Bulk quantization (a whole prompt or cache)
-  // takes several steps of rows per wave.
-  constexpr int RPS = 64 / (D * NB / 64);  // rows per wave and step: 64 / (DP / 8)
-  const bool wide = !((uintptr_t)x & 15) && !((uintptr_t)pk & 7) && rows <= INT32_MAX;
-  if (wide) {
-    const bool bulk = rows >= 65536;
-    const int steps = bulk ? ((8 / ((8 / NB) * (f32 ? 2 : 1))) > 0 ? 8 / ((8 / NB) * (f32 ? 2 : 1)) : 1) : 1;
-    const int per_wg = 4 * RPS * steps;
+  const int64_t rows = (int64_t)B * HKV * N;
+  constexpr int RPS = WideRow<D, NB, GS, false>::RPS;
+  const bool wide = !((uintptr_t)src.x & 15) && !((uintptr_t)pk & 7);
+  const bool bulk = rows >= kBulkRows;
+  const int steps = bulk ? ((8 / ((8 / NB) * (f32 ? 2 : 1))) > 0 ? 8 / ((8 / NB) * (f32 ? 2 : 1)) : 1) : 1;
+  const int per_wg = 4 * RPS * steps;
+  const int64_t tiles = ((int64_t)N + per_wg - 1) / per_wg;
+  if (wide && pm.page_size == 0 && N >= kTokensMinN && B <= 65535 && tiles * HKV <= INT32_MAX / 256 &&
+      !(((uintptr_t)sc | (uintptr_t)zr) & 3)) {
+    const dim3 grid((unsigned)(tiles * HKV), (unsigned)B);
+#define TKV_TOKENS(F, ST) \
+  quantize_tokens_kernel<D, NB, GS, F, ST><<<grid, 256, 0, st>>>(src, HKV, N, (int)tiles, pos, S_cap, pk, sc, zr)
+    constexpr int S16 = 8 / (8 / NB), S32 = 4 / (8 / NB);  // steps of ~128 B per lane
+    if (f32) {
+      if (bulk) TKV_TOKENS(true, (S32 > 0 ? S32 : 1)); else TKV_TOKENS(true, 1);
+    } else {
+      if (bulk) TKV_TOKENS(false, S16); else TKV_TOKENS(false, 1);
+    }
+#undef TKV_TOKENS
+  } else if (wide && rows <= INT32_MAX) {
     const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
     const int r = (int)rows;
 #define TKV_WIDE(F, BK) \
-  quantize_pack_wide_kernel<D, NB, GS, F, BK><<<grid, 256, 0, st>>>(x, r, HKV, N, pos, S_cap, pm, pk, sc, zr)
+  quantize_pack_wide_kernel<D, NB, GS, F, BK><<<grid, 256, 0, st>>>(src.x, r, HKV, N, pos, S_cap, pm, pk, sc, zr)
     if (f32) {
       if (bulk) TKV_WIDE(true, true); else TKV_WIDE(true, false);
     } else {
@@ -519,9 +657,9 @@ static void launch_quantize(const void* x, bool f32, int64_t rows, int HKV, int 
       const int64_t n = rows - row0 < 4 * kMaxBlocks ? rows - row0 : 4 * kMaxBlocks;
       const dim3 grid((unsigned)((n + 3) / 4));
       if (f32)
-        quantize_pack_kernel<D, NB, GS, true><<<grid, 256, 0, st>>>(x, row0, rows, HKV, N, pos, S_cap, pm, pk, sc, zr);
+        quantize_pack_kernel<D, NB, GS, true><<<grid, 256, 0, st>>>(src.x, row0, rows, HKV, N, pos, S_cap, pm, pk, sc, zr);
       else
-        quantize_pack_kernel<D, NB, GS, false><<<grid, 256, 0, st>>>(x, row0, rows, HKV, N, pos, S_cap, pm, pk, sc, zr);
+        quantize_pack_kernel<D, NB, GS, false><<<grid, 256, 0, st>>>(src.x, row0, rows, HKV, N, pos, S_cap, pm, pk, sc, zr);
     }
   }
 }
@@ -583,12 +721,12 @@ extern "C" int tkv_quantize_pack(const void* x, int32_t x_is_fp32, int32_t B, in
   if (!positions && N > S_cap) return TKV_EINVAL;
   if (((uintptr_t)packed & 3) || ((uintptr_t)scale & 1) || ((uintptr_t)zero & 1)) return TKV_EINVAL;
   if ((uintptr_t)x & (x_is_fp32 ? 3 : 1)) return TKV_EINVAL;
-  const int64_t rows = (int64_t)B * HKV * N;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const PageMap pm{nullptr, 0, 0, 0};
+  const TokenSource src{x, (int64_t)HKV * N * D, (int64_t)N * D, D};
   (void)hipGetLastError();
 #define TKV_Q(Dv, NBv, GSv) \
-  launch_quantize<Dv, NBv, GSv>(x, x_is_fp32 != 0, rows, HKV, N, positions, S_cap, pm, packed, scale, zero, st)
+  launch_quantize<Dv, NBv, GSv>(src, x_is_fp32 != 0, B, HKV, N, positions, S_cap, pm, packed, scale, zero, st)
   TKV_DISPATCH_DNG(D, nbits, group_size, TKV_Q);
 #undef TKV_Q
   const hipError_t e = hipGetLastError();
@@ -611,13 +749,13 @@ extern "C" int tkv_paged_quantize_pack(const void* x, int32_t x_is_fp32, int32_t
   if (group_size <= 0 || D % group_size) return TKV_EINVAL;
   if (((uintptr_t)packed & 3) || ((uintptr_t)scale & 1) || ((uintptr_t)zero & 1)) return TKV_EINVAL;
   if ((uintptr_t)x & (x_is_fp32 ? 3 : 1)) return TKV_EINVAL;
-  const int64_t rows = (int64_t)B * HKV * N;
   const int S_cap = block_table_stride * page_size;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const TokenSource src{x, (int64_t)HKV * N * D, (int64_t)N * D, D};
   const PageMap pm{block_table, block_table_stride, page_size, num_pages};
   (void)hipGetLastError();
 #define TKV_Q(Dv, NBv, GSv) \
-  launch_quantize<Dv, NBv, GSv>(x, x_is_fp32 != 0, rows, HKV, N, positions, S_cap, pm, packed, scale, zero, st)
+  launch_quantize<Dv, NBv, GSv>(src, x_is_fp32 != 0, B, HKV, N, positions, S_cap, pm, packed, scale, zero, st)
   TKV_DISPATCH_DNG(D, nbits, group_size, TKV_Q);
 #undef TKV_Q
   const hipError_t e = hipGetLastError();

@@ -129,6 +129,110 @@ __device__ __forceinline__ float rint_quotient(float a, float s, float rs) {
   return q;
 }
 
+// ---------------------------------------------------------------------------
+// The same arithmetic for kernels whose lanes hold many values of a group.
+// ---------------------------------------------------------------------------
+struct GroupScale {
+  float s, z;     // the fp16 scale and zero, as fp32
+  uint32_t bits;  // their fp16 bits: scale low, zero high
+};
+
+// Scale and zero of a group.  The division of the range by the constant QMAX is
+// a product with its reciprocal and one correction step: the same bits as the
+// IEEE quotient for every finite non-negative fp32 range and QMAX 3 and 15
+// (checked over all of them); an infinite or NaN range passes through.
+template <int QMAX>
+__device__ __forceinline__ GroupScale group_scale(float mn, float mx) {
+  constexpr float inv = 1.0f / QMAX;
+  const float range = mx - mn;
+  const float q0 = range * inv;
+  float sc = fmaf(fmaf((float)-QMAX, q0, range), inv, q0);
+  if (!(range < INFINITY)) sc = range;
+  if (!(sc > 0.0f)) sc = 1.0f;
+  const _Float16 s16 = (_Float16)sc, z16 = (_Float16)mn;
+  return GroupScale{(float)s16, (float)z16,
+                    (uint32_t)__builtin_bit_cast(uint16_t, s16) | ((uint32_t)zero_bits(mn) << 16)};
+}
+
+// A code as an integer added into a word.  The quotient of d by an fp16 scale
+// is correctly rounded by one correction step, q1 = RN(q0 + r * rs) with
+// q0 = RN(d * rs) and r = d - q0 * s: with rs within 1 ulp of 1/s, q0 is within
+// 2.5 ulp of d/s, so r fits (s has 11 significant bits) and is exact, and r * rs
+// is off by under 2^-21 ulp of q1, while d/s lies at least 2^-11 ulp from every
+// midpoint of two floats (and on none: an odd 25-bit midpoint times s is no
+// 24-bit number).  q1 + 1.5 * 2^23 then rounds to an integer, ties to even, in
+// the low bits of the sum, whose bits, clamped to those of codes 0..QMAX, are
+// the code plus a constant that code_bias cancels.  A group with an infinite,
+// zero or NaN scale or zero is not for this path (group_special).
+constexpr float kCodeMagic = 12582912.0f;
+constexpr uint32_t kCodeMagicBits = 0x4B400000u;
+
+template <int QMAX>
+__device__ __forceinline__ uint32_t code_term(float d, float s, float rs) {
+  const float q0 = d * rs;
+  const float q1 = fmaf(fmaf(-q0, s, d), rs, q0);
+  const int bits = __builtin_bit_cast(int, q1 + kCodeMagic);
+  return (uint32_t)min(max(bits, (int)kCodeMagicBits), (int)(kCodeMagicBits + QMAX));
+}
+// 0 for an ordinary group, NaN for one whose scale, its reciprocal or its zero
+// is not finite.
+__device__ __forceinline__ float group_special(float s, float z, float rs) {
+  return (s + z + rs) * 0.0f;
+}
+// Start of a word of four bytes of P codes each, so that the terms' constants
+// sum to zero.
+template <int P, int NB>
+__device__ __forceinline__ constexpr uint32_t code_bias() {
+  uint32_t s = 0;
+  for (int e = 0; e < 4; ++e)
+    for (int p = 0; p < P; ++p) s -= kCodeMagicBits << (8 * e + p * NB);
+  return s;
+}
+// The same code by IEEE division and torch's clamp (NaN gives code 0).
+template <int QMAX>
+__device__ __forceinline__ uint32_t code_by_division(float d, float s) {
+  float c = rintf(d / s);
+  if (c != c) c = 0.0f;
+  return (uint32_t)fminf(fmaxf(c, 0.0f), (float)QMAX);
+}
+
+// Half HI of w less z, rounded once (v_fma_mix_f32: the 1.0 is opaque, or the
+// conversion would become an instruction of its own).
+__device__ __forceinline__ float half_less(uint32_t w, bool hi, float z) {
+  float one = 1.0f;
+  asm("" : "+v"(one));
+  const h2 v = __builtin_bit_cast(h2, w);
+  return fmaf((float)(hi ? v[1] : v[0]), one, -z);
+}
+
+// (min, -max) of the eight fp16 values of a 16-byte vector.
+__device__ __forceinline__ h2 run_minmax(u4 v) {
+  h2 x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(h2, (uint32_t)v[i]);
+  const h2 mn = __builtin_elementwise_minimum(
+      __builtin_elementwise_minimum(__builtin_elementwise_minimum(x[0], x[1]), x[2]), x[3]);
+  const h2 mx = -__builtin_elementwise_maximum(
+      __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[0], x[1]), x[2]), x[3]);
+  return __builtin_elementwise_minimum(h2{mn[0], mx[0]}, h2{mn[1], mx[1]});
+}
+template <int CTRL>
+__device__ __forceinline__ h2 pair_min_dpp(h2 v) {
+  const h2 o = __builtin_bit_cast(
+      h2, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+  return __builtin_elementwise_minimum(v, o);
+}
+// Pairwise min over aligned runs of W lanes (W <= 16), as minmax_lanes.
+template <int W>
+__device__ __forceinline__ h2 pair_min_lanes(h2 v) {
+  static_assert(W <= 16, "runs of at most a row of lanes");
+  if constexpr (W >= 2) v = pair_min_dpp<0xB1>(v);
+  if constexpr (W >= 4) v = pair_min_dpp<0x4E>(v);
+  if constexpr (W >= 8) v = pair_min_dpp<0x141>(v);
+  if constexpr (W >= 16) v = pair_min_dpp<0x140>(v);
+  return v;
+}
+
 // x[p] = the row's value at dim (lane % DP) + p * DP, already in fp32.
 template <int D, int NB, int GS>
 __device__ __forceinline__ RowQuant<D, NB, GS> quantize_row(const float (&x)[8 / NB], int lane) {
