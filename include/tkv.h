@@ -251,6 +251,23 @@ int tkv_quantize_keys_channel(const void *x, int32_t x_is_fp32, int32_t B, int32
                               int32_t S_cap, uint8_t *packed, uint16_t *scale, uint16_t *zero,
                               tkv_stream_t stream);
 
+/* A prompt into a per-channel cache whose windows are empty: fp16 k and v, value
+ * d of token t of (b, kv head) at element b * strides[0] + kv * strides[1] +
+ * t * strides[2] + d (any layout with contiguous rows, e.g. the token-major
+ * view a projection leaves; base and strides 16-byte multiples).  The whole
+ * 32-token blocks of the N tokens are quantized into the history at token
+ * `start` (a multiple of 32; start + N <= S_cap) -- keys exactly as
+ * tkv_quantize_keys_channel, values as tkv_quantize_pack -- the rest goes to window rows 0 .., and every row's q_lens becomes
+ * start + whole blocks, its res_lens the rest.  Three launches.  No
+ * counterpart in the reference (it plans the format). */
+int tkv_channel_extend(const void *k, const int64_t *k_strides, const void *v,
+                       const int64_t *v_strides, int32_t B, int32_t HKV, int32_t N, int32_t D,
+                       int32_t k_nbits, int32_t v_nbits, int32_t group_size, int32_t start,
+                       void *k_res, void *v_res, int32_t res_cap, int32_t *q_lens,
+                       int32_t *res_lens, int32_t S_cap, uint8_t *k_packed, uint16_t *k_scale,
+                       uint16_t *k_zero, uint8_t *v_packed, uint16_t *v_scale, uint16_t *v_zero,
+                       tkv_stream_t stream);
+
 /* The fp16 window of per-channel keys, as two launches per decode step that
  * keep every length on the device (so a captured step replays correctly for
  * any window fill).  k_res / v_res: fp16 (B, HKV, res_cap, D) with res_cap

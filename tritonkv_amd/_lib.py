@@ -105,6 +105,8 @@ SIGNATURES = {
                                    _P], ctypes.c_int),
     "tkv_channel_decode_attention": ([ctypes.POINTER(DecodeArgs), _P, _P, _P, _I32, _P],
                                      ctypes.c_int),
+    "tkv_channel_extend": ([_P, _P, _P, _P] + [_I32] * 8 + [_P, _P, _I32, _P, _P, _I32] + [_P] * 7,
+                           ctypes.c_int),
     "tkv_channel_window_append": ([_P, _P, _I32, _I32, _I32, _P, _P, _I32, _P, _P], ctypes.c_int),
     "tkv_channel_window_flush": ([_P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P, _I32,
                                   _P, _P, _P, _P, _P, _P, _P], ctypes.c_int),

@@ -25,6 +25,7 @@ one length for every batch row.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
@@ -204,6 +205,18 @@ def channel_decode_attention(
     return out
 
 
+def _strided_rows(x: torch.Tensor):
+    """``(x, strides)`` of an fp16 ``(B, HKV, N, D)`` tensor as tkv_channel_extend
+    reads it: contiguous rows, base and strides 16-byte multiples.  A view
+    that has those (a token-major projection, a slice of tokens) is read in
+    place, anything else as a contiguous copy."""
+    strides = [st if n > 1 else 0 for n, st in zip(x.shape[:3], x.stride()[:3])]
+    if x.stride(3) != 1 or x.data_ptr() % 16 or any(st % 8 for st in strides):
+        x = x.clone(memory_format=torch.contiguous_format)
+        strides = x.stride()[:3]
+    return x, (ctypes.c_int64 * 3)(*strides)
+
+
 class ChannelKVCache:
     """One layer's cache: per-channel keys, per-token values, fp16 window.
 
@@ -236,8 +249,8 @@ class ChannelKVCache:
         self.quantized = 0   # tokens in the quantized history (a multiple of 32)
         self.window = 0      # tokens in the fp16 window (< 32)
         self._pos = torch.zeros(B, dtype=torch.int32, device=device)
-        self._qlens = torch.zeros(B, dtype=torch.int32, device=device)
-        self._rlens = torch.zeros(B, dtype=torch.int32, device=device)
+        self._lens = torch.zeros(2, B, dtype=torch.int32, device=device)
+        self._qlens, self._rlens = self._lens  # quantized tokens and window fill of each row
         self.workspace: dict = {}
 
     def __len__(self) -> int:
@@ -246,8 +259,7 @@ class ChannelKVCache:
     def reset(self) -> None:
         """Forget every token (host counters and device-side lengths)."""
         self.quantized = self.window = 0
-        self._qlens.zero_()
-        self._rlens.zero_()
+        self._lens.zero_()
 
     def nbytes(self) -> int:
         return self.keys.nbytes() + self.values.nbytes() + 2 * self.k_res.numel() * 2
@@ -278,7 +290,9 @@ class ChannelKVCache:
         self.window = 0
 
     def extend(self, k: torch.Tensor, v: torch.Tensor) -> None:
-        """Append ``(B, HKV, N, D)`` keys and values from the host (prefill)."""
+        """Append ``(B, HKV, N, D)`` keys and values from the host (prefill).
+        With an empty window that is three launches, which read ``k`` and ``v``
+        in the layout they have (rows contiguous, strides 16-byte multiples)."""
         self._check_tokens(k, v)
         if k.dtype != torch.float16:
             k = k.to(torch.float16)
@@ -288,23 +302,37 @@ class ChannelKVCache:
         if len(self) + N > self.capacity:
             raise ValueError(f"cache capacity {self.capacity} exceeded ({len(self)} + {N})")
         i = 0
-        if self.window == 0 and N >= BLOCK:  # whole blocks straight into the history
-            n = (N // BLOCK) * BLOCK
-            self._pos.fill_(self.quantized)
-            append_keys_per_channel(self.keys, k[:, :, :n], self._pos)
-            append_kv(self.values, v[:, :, :n].contiguous(), self._pos)
-            self.quantized += n
-            i = n
-        while i < N:
-            take = min(BLOCK - self.window, N - i)
-            self.k_res[:, :, self.window:self.window + take] = k[:, :, i:i + take]
-            self.v_res[:, :, self.window:self.window + take] = v[:, :, i:i + take]
-            self.window += take
-            i += take
+        if (self.window and N) or not k.is_cuda:  # fill the open window first
+            i = min(BLOCK - self.window, N)
+            self.k_res[:, :, self.window:self.window + i] = k[:, :, :i]
+            self.v_res[:, :, self.window:self.window + i] = v[:, :, :i]
+            self.window += i
             if self.window == BLOCK:
                 self._flush()
-        self._qlens.fill_(self.quantized)
-        self._rlens.fill_(self.window)
+        if i < N:
+            self._extend_empty_window(k[:, :, i:], v[:, :, i:])
+        else:
+            self._qlens.fill_(self.quantized)
+            self._rlens.fill_(self.window)
+
+    def _extend_empty_window(self, k: torch.Tensor, v: torch.Tensor) -> None:
+        """Whole blocks of ``k`` / ``v`` straight into the history, the rest
+        into the (empty) window, the device-side lengths with them."""
+        k, ks = _strided_rows(k)
+        v, vs = _strided_rows(v)
+        B, HKV, N, D = k.shape
+        kc, vc = self.keys, self.values
+        with torch.cuda.device(self.k_res.device):
+            rc = _lib.load().tkv_channel_extend(
+                k.data_ptr(), ks, v.data_ptr(), vs, B, HKV, N, D, kc.nbits, vc.nbits,
+                vc.group_size, self.quantized, self.k_res.data_ptr(), self.v_res.data_ptr(), BLOCK,
+                self._qlens.data_ptr(), self._rlens.data_ptr(), self.capacity,
+                kc.packed.data_ptr(), kc.scale.data_ptr(), kc.zero.data_ptr(),
+                vc.packed.data_ptr(), vc.scale.data_ptr(), vc.zero.data_ptr(),
+                _lib.stream_handle(self.k_res.device))
+            _lib.check(rc, "ChannelKVCache.extend")
+        self.quantized += N // BLOCK * BLOCK
+        self.window = N % BLOCK
 
     def attend(self, q: torch.Tensor, sm_scale: float | None = None,
                out: torch.Tensor | None = None) -> torch.Tensor:

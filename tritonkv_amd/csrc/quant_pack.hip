@@ -217,7 +217,7 @@ quantize_pack_wide_kernel(const void* __restrict__ x, int rows, int HKV, int N,
                           uint16_t* __restrict__ zero) {
   using W = WideRow<D, NB, GS, F32>;
   constexpr int P = W::P, DP = W::DP, NG = W::NG, RPS = W::RPS;
-  constexpr int STEPS = BULK ? (8 / (P * W::NV) > 0 ? 8 / (P * W::NV) : 1) : 1;  // ~128 B per lane
+  constexpr int STEPS = BULK && 8 / (P * W::NV) > 0 ? 8 / (P * W::NV) : 1;  // ~128 B per lane
 
   const int lane = threadIdx.x & 63, slot = lane / W::LPR, c = lane % W::LPR;
   const int first = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * STEPS * RPS;
@@ -271,7 +271,7 @@ quantize_pack_wide_kernel(const void* __restrict__ x, int rows, int HKV, int N,
 template <int D, int NB, int GS, bool F32, int STEPS>
 __global__ void __launch_bounds__(256)
 quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
-                       const int32_t* __restrict__ positions, int S_cap,
+                       const int32_t* __restrict__ positions, int start, int S_cap,
                        uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
                        uint16_t* __restrict__ zero) {
   using W = WideRow<D, NB, GS, F32>;
@@ -294,7 +294,7 @@ quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
 
   // Token t0 + i of the wave goes to row dst0 + i of the (b, kv head) block; rows
   // i in [lo, hi) exist and fit the capacity.
-  const int64_t dst0 = (int64_t)(positions ? positions[b] : 0) + t0;
+  const int64_t dst0 = (int64_t)(positions ? positions[b] : start) + t0;
   const int64_t left = max((int64_t)S_cap - dst0, (int64_t)0);
   const int lo = (int)min(max(-dst0, (int64_t)0), (int64_t)ROWS);
   const int hi = (int)min((int64_t)min(ROWS, N - t0), left);
@@ -334,85 +334,244 @@ quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
   }
 }
 
-// Per-channel (KIVI-style) keys.  One wave quantizes one block of 32 tokens
-// of one (b, kv head): every channel of the block is one group of 32 values
-// (min/max, fp16 scale and zero, codes), the group-wise arithmetic of
-// quantize_row applied along the token axis.  Lane j owns byte column j of
-// the block's rows, i.e. channels j + p*DP (p < P), so the min/max need no
-// cross-lane step and the lane packs each token's byte j itself.  Lanes >= DP
-// repeat lanes j - DP and store nothing.
-//   src: element index of the block's first row in x (rows D apart);
-//   dst_row: the block's first destination row in packed;
-//   meta: element index of the block's scale / zero row (D values).
+// Per-channel (KIVI-style) keys.  A block of 32 tokens of one (b, kv head) is
+// quantized by D / 2 lanes of a wave: every channel of the block is one group of
+// 32 values (min/max, fp16 scale and zero, codes), the group-wise arithmetic
+// of quantize_row applied along the token axis.  Lane j of the block owns
+// channels 2j and 2j + 1, so a token's row is one contiguous load (256 bytes at
+// D = 128 fp16), the min/max need no cross-lane step, and scale and zero leave
+// as whole dwords.  A byte column's P channels sit in P lanes LS = DP / 2
+// apart: each lane packs its codes of two tokens into a dword at its slice's
+// bits, an OR-reduction over those lanes by lane swaps leaves every lane
+// 16 / P of the dwords, and two exchanges with neighbouring lanes turn them into
+// 8-byte pieces of packed rows.
+// Bound by HBM: 4 x 8 heads of 8192 tokens, D = 128, fp16 to 2-bit, from a
+// token-major source: 18.1 us (4.5 TB/s); byte columns per lane (2-byte loads,
+// byte stores) took 35.9 us after a 36.4 us copy to contiguous keys.
 template <int D, int NB, bool F32>
-__device__ __forceinline__ void quantize_key_block(const void* __restrict__ x, int64_t src, int lane,
-                                                   bool ok, uint8_t* __restrict__ packed,
-                                                   int64_t dst_row, uint16_t* __restrict__ scale,
-                                                   uint16_t* __restrict__ zero, int64_t meta) {
-  constexpr int P = 8 / NB, DP = D / P, QMAX = (1 << NB) - 1, T = 32;
-  const int j = lane % DP;
-  ok = ok && lane < DP;
-  float v[P][T];
+struct KeyBlock {
+  static constexpr int P = 8 / NB, DP = D / P, QMAX = (1 << NB) - 1, T = 32;
+  static constexpr int LB = D / 2;          // lanes of a block
+  static constexpr int BPW = 64 / LB;       // blocks per wave
+  static constexpr int LS = DP / 2;         // lanes of a slice
+  static constexpr int NW = T / 2;          // dwords of codes per lane: two tokens each
+  static constexpr int NR = NW / P;         // ... after the reduction over the slices
+
+  // x: the first row of the block, rows st elements apart (wide: pairs of
+  // channels may be read as one aligned load); packed: the block's first row;
+  // scale / zero: its D values; ok: whether this lane's block is stored.
+  __device__ static void quantize(const void* __restrict__ x, int64_t st, bool wide, int lane,
+                                  bool ok, uint8_t* __restrict__ packed,
+                                  uint16_t* __restrict__ scale, uint16_t* __restrict__ zero) {
+    const int j = lane % LB;
+    uint32_t raw[T][F32 ? 2 : 1];
+    if (wide) {
 #pragma unroll
-  for (int t = 0; t < T; ++t)
+      for (int t = 0; t < T; ++t) {
+        if constexpr (F32) {
+          const u2 v = __builtin_nontemporal_load(
+              reinterpret_cast<const u2*>(static_cast<const float*>(x) + t * st + 2 * j));
+          raw[t][0] = v[0];
+          raw[t][1] = v[1];
+        } else {
+          raw[t][0] = __builtin_nontemporal_load(
+              reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(x) + t * st + 2 * j));
+        }
+      }
+    } else {
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int64_t e = src + (int64_t)t * D + j + p * DP;
-      v[p][t] = F32 ? static_cast<const float*>(x)[e] : (float)static_cast<const _Float16*>(x)[e];
+      for (int t = 0; t < T; ++t) {
+        if constexpr (F32) {
+          const uint32_t* v = static_cast<const uint32_t*>(x) + t * st + 2 * j;
+          raw[t][0] = v[0];
+          raw[t][1] = v[1];
+        } else {
+          const uint16_t* v = static_cast<const uint16_t*>(x) + t * st + 2 * j;
+          raw[t][0] = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
+        }
+      }
     }
-  uint32_t bytes[T];
+    float mn[2], mx[2];
+    if constexpr (F32) {
 #pragma unroll
-  for (int t = 0; t < T; ++t) bytes[t] = 0;
+      for (int c = 0; c < 2; ++c) {
+        mn[c] = mx[c] = as_float(raw[0][c]);
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    float mn = v[p][0], mx = v[p][0];
+        for (int t = 1; t < T; ++t) {
+          mn[c] = nan_min(mn[c], as_float(raw[t][c]));
+          mx[c] = nan_max(mx[c], as_float(raw[t][c]));
+        }
+      }
+    } else {
+      h2 lo = __builtin_bit_cast(h2, raw[0][0]), hi = lo;
 #pragma unroll
-    for (int t = 1; t < T; ++t) {
-      mn = nan_min(mn, v[p][t]);
-      mx = nan_max(mx, v[p][t]);
+      for (int t = 1; t < T; ++t) {
+        lo = __builtin_elementwise_minimum(lo, __builtin_bit_cast(h2, raw[t][0]));
+        hi = __builtin_elementwise_maximum(hi, __builtin_bit_cast(h2, raw[t][0]));
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) mn[c] = (float)lo[c], mx[c] = (float)hi[c];
     }
-    float sc = (mx - mn) / (float)QMAX;
-    if (!(sc > 0.0f)) sc = 1.0f;
-    const _Float16 s16 = (_Float16)sc;
-    const _Float16 z16 = (_Float16)mn;
-    const float sf = (float)s16, zf = (float)z16, rs = __builtin_amdgcn_rcpf(sf);
+    uint32_t w[NW], bits[2];
+    float sf[2], zf[2], special = 0.0f;
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-      float c = rint_quotient(v[p][t] - zf, sf, rs);
-      if (c != c) c = 0.0f;
-      c = fminf(fmaxf(c, 0.0f), (float)QMAX);
-      bytes[t] |= (uint32_t)c << (p * NB);
+    for (int k = 0; k < NW; ++k) w[k] = code_bias<1, NB>();
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const GroupScale g = group_scale<QMAX>(mn[c], mx[c]);
+      bits[c] = g.bits;
+      sf[c] = g.s;
+      zf[c] = g.z;
+      const float rs = __builtin_amdgcn_rcpf(g.s);
+      special += group_special(g.s, g.z, rs);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        w[t / 2] += code_term<QMAX>(less(raw[t], c, g.z), g.s, rs) << (16 * (t & 1) + 8 * c);
+    }
+    if (__builtin_expect(special != 0.0f, 0)) {  // NaN: redo the lane's codes by division
+#pragma unroll
+      for (int k = 0; k < NW; ++k) w[k] = 0;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          w[t / 2] |= code_by_division<QMAX>(less(raw[t], c, zf[c]), sf[c]) << (16 * (t & 1) + 8 * c);
+    }
+    // Dword k of lane j: tokens 2k, 2k + 1 (low, high half) at slice j / LS's bits.
+    const int shift = (j / LS) * NB;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) w[k] <<= shift;
+    // OR over the lanes of a byte column; each step leaves a lane half of its
+    // dwords, the upper half where the lane's bit is set.
+    int k0 = 0;  // index of dword 0
+    if constexpr (D == 128) {
+      or_scatter<32, NW>(w, lane, k0);
+      if constexpr (P == 4) or_scatter<16, NW / 2>(w, lane, k0);
+    } else {
+      or_scatter<16, NW>(w, lane, k0);
+      if constexpr (P == 4) or_scatter<8, NW / 2>(w, lane, k0);
     }
     if (ok) {
-      scale[meta + j + p * DP] = __builtin_bit_cast(uint16_t, s16);
-      zero[meta + j + p * DP] = zero_bits(mn);
+      if (!(((uintptr_t)scale | (uintptr_t)zero) & 3)) {
+        reinterpret_cast<uint32_t*>(scale)[j] = perm(bits[1], bits[0], 0x05040100u);
+        reinterpret_cast<uint32_t*>(zero)[j] = perm(bits[1], bits[0], 0x07060302u);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          scale[2 * j + c] = (uint16_t)bits[c];
+          zero[2 * j + c] = (uint16_t)(bits[c] >> 16);
+        }
+      }
+    }
+    // Lanes j, j ^ 1 hold adjacent byte pairs of two tokens each: the even lane
+    // takes the four bytes of token 2k, the odd one those of 2k + 1.
+    const bool odd = lane & 1, upper = lane & 2;
+    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) w[k] = perm(dpp<0xB1>(w[k]), w[k], sel);
+    // Lanes j, j ^ 2 then hold adjacent dwords: the lower takes 8 bytes of even
+    // dwords' tokens, the upper of odd ones'.
+    const int col = 8 * ((j % LS) >> 2);
+#pragma unroll
+    for (int i = 0; i < NR / 2; ++i) {
+      const uint32_t got = dpp<0x4E>(upper ? w[2 * i] : w[2 * i + 1]);
+      const u2 v = upper ? u2{got, w[2 * i + 1]} : u2{w[2 * i], got};
+      const int t = 2 * (k0 + 2 * i + (upper ? 1 : 0)) + (odd ? 1 : 0);
+      if (!ok) continue;
+      uint8_t* dst = packed + t * DP + col;
+      if (!((uintptr_t)packed & 7)) {
+        *reinterpret_cast<u2*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dst[e] = (uint8_t)(v[e / 4] >> (8 * (e % 4)));
+      }
     }
   }
-  if (!ok) return;
-#pragma unroll
-  for (int t = 0; t < T; ++t) packed[(dst_row + t) * DP + j] = (uint8_t)bytes[t];
-}
 
-// One wave per block of 32 tokens of one (b, kv head).  A block whose
-// destination does not start on a 32-token boundary, or does not fit
-// [0, S_cap), is not written.
+ private:
+  __device__ static float as_float(uint32_t v) { return __builtin_bit_cast(float, v); }
+  __device__ static float less(const uint32_t (&raw)[F32 ? 2 : 1], int c, float z) {
+    if constexpr (F32) return as_float(raw[c]) - z;
+    else return half_less(raw[0], c, z);
+  }
+  template <int CTRL>
+  __device__ static uint32_t dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+  }
+  // w[0 .. N/2) = the OR over lanes l and l ^ X of w[k] (bit X of l clear) or
+  // w[k + N/2] (set).
+  template <int X, int N>
+  __device__ static void or_scatter(uint32_t (&w)[NW], int lane, int& k0) {
+    const bool set = lane & X;
+#pragma unroll
+    for (int k = 0; k < N / 2; ++k) {
+      if constexpr (X == 8) {
+        const uint32_t keep = set ? w[k + N / 2] : w[k], send = set ? w[k] : w[k + N / 2];
+        w[k] = keep | dpp<0x128>(send);
+      } else {
+        // the swap leaves (own, partner's) halves of w[k] in the clear lanes
+        // and of w[k + N/2] in the set ones
+        const auto s = X == 32 ? __builtin_amdgcn_permlane32_swap(w[k], w[k + N / 2], false, false)
+                               : __builtin_amdgcn_permlane16_swap(w[k], w[k + N / 2], false, false);
+        w[k] = opaque(s[0]) | opaque(s[1]);
+      }
+    }
+    if (set) k0 += N / 2;
+  }
+};
+
+// A block whose destination does not start on a 32-token boundary, or does not
+// fit [0, S_cap), is not written.  Blocks of a batch row are dealt to waves
+// heads first for a token-major source (neighbouring waves then read
+// neighbouring memory), tokens first otherwise.
 template <int D, int NB, bool F32>
 __global__ void __launch_bounds__(256)
-quantize_keys_channel_kernel(const void* __restrict__ x, int64_t blocks, int HKV, int NBLK,
-                             const int32_t* __restrict__ positions, int S_cap,
+quantize_keys_channel_kernel(TokenSource src, bool wide, int B, int HKV, int NBLK,
+                             const int32_t* __restrict__ positions, int start, int S_cap,
                              uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
                              uint16_t* __restrict__ zero) {
-  constexpr int T = 32;
+  using K = KeyBlock<D, NB, F32>;
+  constexpr int T = K::T;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t blk = (int64_t)blockIdx.x * 4 + w;
-  if (blk >= blocks) return;  // whole wave
-  const int64_t bh = blk / NBLK;
-  const int tb = (int)(blk - bh * NBLK);
-  const int b = (int)(bh / HKV);
-  const int64_t dst_t = (int64_t)(positions ? positions[b] : 0) + (int64_t)tb * T;
-  const bool ok = dst_t >= 0 && dst_t % T == 0 && dst_t + T <= S_cap;
-  quantize_key_block<D, NB, F32>(x, (bh * NBLK + tb) * T * D, lane, ok, packed, bh * S_cap + dst_t,
-                                 scale, zero, (bh * (S_cap / T) + dst_t / T) * D);
+  const int first = ((int)blockIdx.x * 4 + w) * K::BPW, blocks = HKV * NBLK;
+  if (first >= blocks) return;  // whole wave
+  const int i = first + (K::BPW > 1 ? lane / K::LB : 0);
+  const int ii = min(i, blocks - 1);
+  const bool heads_first = src.st != D;
+  const int q = ii / (heads_first ? HKV : NBLK), m = ii - q * (heads_first ? HKV : NBLK);
+  const int kv = heads_first ? m : q, tb = heads_first ? q : m;
+  for (int b = blockIdx.y; b < B; b += gridDim.y) {
+    const int64_t off = b * src.sb + kv * src.sh + (int64_t)tb * T * src.st;
+    const int64_t dst_t = (int64_t)(positions ? positions[b] : start) + (int64_t)tb * T;
+    const bool ok = i < blocks && dst_t >= 0 && dst_t % T == 0 && dst_t + T <= S_cap;
+    const int64_t bh = (int64_t)b * HKV + kv;
+    const int64_t meta = ok ? (bh * (S_cap / T) + dst_t / T) * D : 0;
+    K::quantize(F32 ? (const void*)(static_cast<const float*>(src.x) + off)
+                    : (const void*)(static_cast<const uint16_t*>(src.x) + off),
+                src.st, wide, lane, ok, packed + (ok ? (bh * S_cap + dst_t) * K::DP : 0),
+                scale + meta, zero + meta);
+  }
+}
+
+// The tokens of a prompt past its last whole block into the window, rows
+// [0, rest) of every (b, kv head), and the batch row's lengths.
+__global__ void __launch_bounds__(256)
+channel_tail_kernel(TokenSource ks, TokenSource vs, int rest, int D, uint16_t* __restrict__ k_res,
+                    uint16_t* __restrict__ v_res, int32_t* __restrict__ q_lens,
+                    int32_t* __restrict__ res_lens, int q_len) {
+  constexpr int T = 32;
+  const int kv = blockIdx.x, b = blockIdx.y, n = rest * D / 8;  // 16-byte vectors per tensor
+  for (int i = threadIdx.x; i < 2 * n; i += blockDim.x) {
+    const TokenSource& s = i < n ? ks : vs;
+    const int e = (i < n ? i : i - n) * 8, t = e / D, d = e % D;
+    const uint16_t* from = static_cast<const uint16_t*>(s.x) + b * s.sb + kv * s.sh + t * s.st + d;
+    uint16_t* to = (i < n ? k_res : v_res) + (((int64_t)b * gridDim.x + kv) * T + t) * D + d;
+    *reinterpret_cast<u4*>(to) = *reinterpret_cast<const u4*>(from);
+  }
+  if (kv == 0 && threadIdx.x == 0) {
+    q_lens[b] = q_len;
+    res_lens[b] = rest;
+  }
 }
 
 // The fp16 window of per-channel keys: K and V windows (B, HKV, 32, D), row b
@@ -440,8 +599,8 @@ channel_window_append_kernel(const uint16_t* __restrict__ k_new, const uint16_t*
 }
 
 // Flush: one workgroup per batch row; if its window holds 32 tokens, wave w
-// quantizes the blocks of kv heads w, w + 4, ...: keys per channel
-// (quantize_key_block), values per token (quantize_row, as the append kernel)
+// quantizes the blocks of kv heads w, w + 4, ...: keys per channel (KeyBlock;
+// lanes past the block's repeat it), values per token (quantize_row, as the append kernel)
 // into the history at q_lens[b]; then q_lens[b] += 32 and res_lens[b] = 0.
 // A window that does not fit the history ([q, q + 32) outside [0, S_cap)) is
 // not written and the lengths do not move: res_lens[b] becomes 33, the
@@ -465,11 +624,12 @@ channel_window_flush_kernel(const uint16_t* __restrict__ k_res, const uint16_t* 
     if (threadIdx.x == 0) res_lens[b] = T + 1;
     return;
   }
-  const bool ok = true;
+  using K = KeyBlock<D, KNB, false>;
+  const bool wide = !((uintptr_t)k_res & 3);
   for (int kv = w; kv < HKV; kv += 4) {
-    const int64_t bh = (int64_t)b * HKV + kv;
-    quantize_key_block<D, KNB, false>(k_res, bh * T * D, lane, ok, kp, bh * S_cap + q, ks, kz,
-                                      (bh * (S_cap / T) + q / T) * D);
+    const int64_t bh = (int64_t)b * HKV + kv, meta = (bh * (S_cap / T) + q / T) * D;
+    K::quantize(k_res + bh * T * D, D, wide, lane, lane < K::LB, kp + (bh * S_cap + q) * K::DP,
+                ks + meta, kz + meta);
     for (int t = 0; t < T; ++t) {
       float x[R::P];
       load_row_for_quant<D, VNB>(v_res + (bh * T + t) * D, false, lane, x);
@@ -615,30 +775,50 @@ constexpr int kTokensMinN = 32;
 // per wave, at most eight waves for each of the chip's 1024 SIMDs.
 constexpr int64_t kBulkRows = 65536;
 
+// Steps of rows per wave: ~128 bytes of input per lane when there are many.
+template <int NB>
+static constexpr int quantize_steps(bool f32, bool bulk) {
+  const int per = (8 / NB) * (f32 ? 2 : 1);  // 16-byte loads per lane and step
+  return bulk && 8 / per > 0 ? 8 / per : 1;
+}
+
+// quantize_tokens_kernel for what it takes; false (nothing launched) otherwise.
+template <int D, int NB, int GS>
+static bool launch_tokens(const TokenSource& src, bool f32, int B, int HKV, int N,
+                          const int32_t* pos, int start, int S_cap, uint8_t* pk, uint16_t* sc,
+                          uint16_t* zr, hipStream_t st) {
+  const int es = f32 ? 4 : 2;
+  const uintptr_t align = (uintptr_t)src.x | (uintptr_t)(src.sb * es) | (uintptr_t)(src.sh * es) |
+                          (uintptr_t)(src.st * es);
+  if ((align & 15) || ((uintptr_t)pk & 7) || (((uintptr_t)sc | (uintptr_t)zr) & 3)) return false;
+  const bool bulk = (int64_t)B * HKV * N >= kBulkRows;
+  const int per_wg = 4 * WideRow<D, NB, GS, false>::RPS * quantize_steps<NB>(f32, bulk);
+  const int64_t tiles = ((int64_t)N + per_wg - 1) / per_wg;
+  if (N < kTokensMinN || B > 65535 || tiles * HKV > INT32_MAX / 256) return false;
+  const dim3 grid((unsigned)(tiles * HKV), (unsigned)B);
+#define TKV_TOKENS(F, BK)                                                                       \
+  quantize_tokens_kernel<D, NB, GS, F, quantize_steps<NB>(F, BK)><<<grid, 256, 0, st>>>(        \
+      src, HKV, N, (int)tiles, pos, start, S_cap, pk, sc, zr)
+  if (f32) {
+    if (bulk) TKV_TOKENS(true, true); else TKV_TOKENS(true, false);
+  } else {
+    if (bulk) TKV_TOKENS(false, true); else TKV_TOKENS(false, false);
+  }
+#undef TKV_TOKENS
+  return true;
+}
+
 template <int D, int NB, int GS>
 static void launch_quantize(const TokenSource& src, bool f32, int B, int HKV, int N,
                             const int32_t* pos, int S_cap, PageMap pm, uint8_t* pk, uint16_t* sc,
                             uint16_t* zr, hipStream_t st) {
+  if (pm.page_size == 0 && launch_tokens<D, NB, GS>(src, f32, B, HKV, N, pos, 0, S_cap, pk, sc, zr, st))
+    return;
   const int64_t rows = (int64_t)B * HKV * N;
-  constexpr int RPS = WideRow<D, NB, GS, false>::RPS;
   const bool wide = !((uintptr_t)src.x & 15) && !((uintptr_t)pk & 7);
-  const bool bulk = rows >= kBulkRows;
-  const int steps = bulk ? ((8 / ((8 / NB) * (f32 ? 2 : 1))) > 0 ? 8 / ((8 / NB) * (f32 ? 2 : 1)) : 1) : 1;
-  const int per_wg = 4 * RPS * steps;
-  const int64_t tiles = ((int64_t)N + per_wg - 1) / per_wg;
-  if (wide && pm.page_size == 0 && N >= kTokensMinN && B <= 65535 && tiles * HKV <= INT32_MAX / 256 &&
-      !(((uintptr_t)sc | (uintptr_t)zr) & 3)) {
-    const dim3 grid((unsigned)(tiles * HKV), (unsigned)B);
-#define TKV_TOKENS(F, ST) \
-  quantize_tokens_kernel<D, NB, GS, F, ST><<<grid, 256, 0, st>>>(src, HKV, N, (int)tiles, pos, S_cap, pk, sc, zr)
-    constexpr int S16 = 8 / (8 / NB), S32 = 4 / (8 / NB);  // steps of ~128 B per lane
-    if (f32) {
-      if (bulk) TKV_TOKENS(true, (S32 > 0 ? S32 : 1)); else TKV_TOKENS(true, 1);
-    } else {
-      if (bulk) TKV_TOKENS(false, S16); else TKV_TOKENS(false, 1);
-    }
-#undef TKV_TOKENS
-  } else if (wide && rows <= INT32_MAX) {
+  if (wide && rows <= INT32_MAX) {
+    const bool bulk = rows >= kBulkRows;
+    const int per_wg = 4 * WideRow<D, NB, GS, false>::RPS * quantize_steps<NB>(f32, bulk);
     const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
     const int r = (int)rows;
 #define TKV_WIDE(F, BK) \
@@ -662,6 +842,38 @@ static void launch_quantize(const TokenSource& src, bool f32, int B, int HKV, in
         quantize_pack_kernel<D, NB, GS, false><<<grid, 256, 0, st>>>(src.x, row0, rows, HKV, N, pos, S_cap, pm, pk, sc, zr);
     }
   }
+}
+
+template <int D, int NB, bool F32>
+static void launch_key_blocks(const TokenSource& src, int B, int HKV, int nblk, const int32_t* pos,
+                              int start, int S_cap, uint8_t* pk, uint16_t* sc, uint16_t* zr,
+                              hipStream_t st) {
+  constexpr int per_wg = 4 * KeyBlock<D, NB, F32>::BPW;
+  constexpr int pair = F32 ? 8 : 4;  // bytes of a lane's two channels
+  const uintptr_t align = (uintptr_t)src.x | (uintptr_t)(src.sb * pair / 2) |
+                          (uintptr_t)(src.sh * pair / 2) | (uintptr_t)(src.st * pair / 2);
+  const dim3 grid((unsigned)(((int64_t)HKV * nblk + per_wg - 1) / per_wg), (unsigned)(B < 65535 ? B : 65535));
+  quantize_keys_channel_kernel<D, NB, F32><<<grid, 256, 0, st>>>(
+      src, !(align & (pair - 1)), B, HKV, nblk, pos, start, S_cap, pk, sc, zr);
+}
+
+static int launch_keys_channel(const TokenSource& src, bool f32, int B, int HKV, int nblk, int D,
+                               int nbits, const int32_t* pos, int start, int S_cap, uint8_t* pk,
+                               uint16_t* sc, uint16_t* zr, hipStream_t st) {
+#define TKV_KC(Dv, NBv)                                                                              \
+  do {                                                                                               \
+    if (f32) launch_key_blocks<Dv, NBv, true>(src, B, HKV, nblk, pos, start, S_cap, pk, sc, zr, st); \
+    else launch_key_blocks<Dv, NBv, false>(src, B, HKV, nblk, pos, start, S_cap, pk, sc, zr, st);    \
+  } while (0)
+  if (D == 128) {
+    if (nbits == 4) TKV_KC(128, 4); else TKV_KC(128, 2);
+  } else if (D == 64) {
+    if (nbits == 4) TKV_KC(64, 4); else TKV_KC(64, 2);
+  } else {
+    return TKV_EUNSUPPORTED;
+  }
+#undef TKV_KC
+  return TKV_OK;
 }
 
 template <int D, int NB, int GS>
@@ -775,28 +987,75 @@ extern "C" int tkv_quantize_keys_channel(const void* x, int32_t x_is_fp32, int32
   if (nbits != 2 && nbits != 4) return TKV_EINVAL;
   if (((uintptr_t)scale & 1) || ((uintptr_t)zero & 1)) return TKV_EINVAL;
   if ((uintptr_t)x & (x_is_fp32 ? 3 : 1)) return TKV_EINVAL;
-  const int64_t blocks = (int64_t)B * HKV * (N / T);
+  if ((int64_t)HKV * (N / T) > INT32_MAX) return TKV_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)((blocks + 3) / 4));
-  const bool f32 = x_is_fp32 != 0;
+  const TokenSource src{x, (int64_t)HKV * N * D, (int64_t)N * D, D};
   (void)hipGetLastError();
-#define TKV_KC(Dv, NBv)                                                                       \
-  do {                                                                                        \
-    if (f32)                                                                                  \
-      quantize_keys_channel_kernel<Dv, NBv, true><<<grid, 256, 0, st>>>(                      \
-          x, blocks, HKV, N / T, positions, S_cap, packed, scale, zero);                      \
-    else                                                                                      \
-      quantize_keys_channel_kernel<Dv, NBv, false><<<grid, 256, 0, st>>>(                     \
-          x, blocks, HKV, N / T, positions, S_cap, packed, scale, zero);                      \
-  } while (0)
-  if (D == 128) {
-    if (nbits == 4) TKV_KC(128, 4); else TKV_KC(128, 2);
-  } else if (D == 64) {
-    if (nbits == 4) TKV_KC(64, 4); else TKV_KC(64, 2);
-  } else {
-    return TKV_EUNSUPPORTED;
+  const int rc = launch_keys_channel(src, x_is_fp32 != 0, B, HKV, N / T, D, nbits, positions, 0,
+                                     S_cap, packed, scale, zero, st);
+  if (rc) return rc;
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? TKV_OK : (int)e;
+}
+
+extern "C" int tkv_channel_extend(const void* k, const int64_t* k_strides, const void* v,
+                                  const int64_t* v_strides, int32_t B, int32_t HKV, int32_t N,
+                                  int32_t D, int32_t k_nbits, int32_t v_nbits, int32_t group_size,
+                                  int32_t start, void* k_res, void* v_res, int32_t res_cap,
+                                  int32_t* q_lens, int32_t* res_lens, int32_t S_cap,
+                                  uint8_t* k_packed, uint16_t* k_scale, uint16_t* k_zero,
+                                  uint8_t* v_packed, uint16_t* v_scale, uint16_t* v_zero,
+                                  tkv_stream_t stream) {
+  using namespace tkv;
+  constexpr int T = 32;
+  if (!k || !v || !k_strides || !v_strides || !k_res || !v_res || !q_lens || !res_lens || !k_packed ||
+      !k_scale || !k_zero || !v_packed || !v_scale || !v_zero)
+    return TKV_EINVAL;
+  if (B <= 0 || HKV <= 0 || N <= 0 || S_cap <= 0 || S_cap % T || res_cap != T) return TKV_EINVAL;
+  if (start < 0 || start % T || (int64_t)start + N > S_cap) return TKV_EINVAL;
+  if ((k_nbits != 2 && k_nbits != 4) || (v_nbits != 2 && v_nbits != 4)) return TKV_EINVAL;
+  if (D != 64 && D != 128) return TKV_EUNSUPPORTED;
+  if (group_size != 16 && group_size != 32 && group_size != 64 && group_size != D) return TKV_EUNSUPPORTED;
+  const TokenSource ks{k, k_strides[0], k_strides[1], k_strides[2]};
+  const TokenSource vs{v, v_strides[0], v_strides[1], v_strides[2]};
+  uintptr_t align = (uintptr_t)k | (uintptr_t)v | (uintptr_t)k_res | (uintptr_t)v_res;
+  for (int i = 0; i < 3; ++i) align |= (uintptr_t)(2 * k_strides[i]) | (uintptr_t)(2 * v_strides[i]);
+  if ((align & 15) || (((uintptr_t)k_packed | (uintptr_t)v_packed) & 7) ||
+      (((uintptr_t)k_scale | (uintptr_t)k_zero | (uintptr_t)v_scale | (uintptr_t)v_zero) & 3))
+    return TKV_EINVAL;
+  const int whole = N / T * T;
+  if ((int64_t)HKV * (whole / T) > INT32_MAX / 256) return TKV_EINVAL;
+  constexpr int kMaxB = 65535;  // a grid's y limit: more batch rows go in pieces
+  for (int b0 = 0; B > kMaxB && b0 < B; b0 += kMaxB) {
+    const int64_t r = (int64_t)b0 * HKV;
+    const int rc = tkv_channel_extend(
+        static_cast<const uint16_t*>(k) + b0 * k_strides[0], k_strides,
+        static_cast<const uint16_t*>(v) + b0 * v_strides[0], v_strides, B - b0 < kMaxB ? B - b0 : kMaxB,
+        HKV, N, D, k_nbits, v_nbits, group_size, start, static_cast<uint16_t*>(k_res) + r * T * D,
+        static_cast<uint16_t*>(v_res) + r * T * D, res_cap, q_lens + b0, res_lens + b0, S_cap,
+        k_packed + r * S_cap * (D * k_nbits / 8), k_scale + r * (S_cap / T) * D,
+        k_zero + r * (S_cap / T) * D, v_packed + r * S_cap * (D * v_nbits / 8),
+        v_scale + r * S_cap * (D / group_size), v_zero + r * S_cap * (D / group_size), stream);
+    if (rc || b0 + kMaxB >= B) return rc;
   }
-#undef TKV_KC
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  (void)hipGetLastError();
+  if (whole) {
+    const int rc = launch_keys_channel(ks, false, B, HKV, whole / T, D, k_nbits, nullptr, start, S_cap,
+                                       k_packed, k_scale, k_zero, st);
+    if (rc) return rc;
+    bool done = false;
+#define TKV_VT(Dv, NBv, GSv) \
+  done = launch_tokens<Dv, NBv, GSv>(vs, false, B, HKV, whole, nullptr, start, S_cap, v_packed, v_scale, v_zero, st)
+    TKV_DISPATCH_DNG(D, v_nbits, group_size, TKV_VT);
+#undef TKV_VT
+    if (!done) return TKV_EINVAL;
+  }
+  const TokenSource kt{static_cast<const uint16_t*>(k) + whole * ks.st, ks.sb, ks.sh, ks.st};
+  const TokenSource vt{static_cast<const uint16_t*>(v) + whole * vs.st, vs.sb, vs.sh, vs.st};
+  channel_tail_kernel<<<dim3((unsigned)HKV, (unsigned)B), 256, 0, st>>>(
+      kt, vt, N - whole, D, static_cast<uint16_t*>(k_res), static_cast<uint16_t*>(v_res), q_lens,
+      res_lens, start + whole);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? TKV_OK : (int)e;
 }
