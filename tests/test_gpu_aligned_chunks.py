@@ -1,0 +1,66 @@
+"""Decode over caches whose blocks start inside a cache line (S no multiple of 32).
+
+Splits of 4096 tokens or more then count their chunks from a multiple of 32
+rows of the tensor and mask the rows before the split: the chunk before the
+block's start (read as zeros), before a later split's start (the previous
+split's rows), and a first chunk that is also the last, with and without the
+appended token in it.  Against the oracle's fp32 attention over the same codes.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tests.helpers import assert_close_to_reference, make_case, oracle_attention_on_quant
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+CASES = [  # nbits, gs, HQ, HKV, D, S, num_splits
+    (4, 32, 8, 2, 128, 4127, 1),     # one tile at a time
+    (4, 32, 8, 2, 128, 8250, 2),     # a second split that starts at a block of 64
+    (4, 32, 12, 2, 128, 8251, 1),    # paired tiles
+    (2, 32, 8, 2, 128, 8263, 1),     # 12 waves
+    (2, 128, 8, 2, 128, 8250, 1),    # one group per row, pairs of metadata
+    (2, 128, 8, 2, 128, 8251, 1),    # ... odd S: not aligned
+    (4, 16, 32, 2, 128, 4099, 1),    # 16 head columns
+    (2, 64, 4, 2, 64, 8199, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_unaligned_blocks_match_the_oracle(case):
+    from tritonkv_amd.kernels import fused_decode_attention
+
+    nbits, gs, HQ, HKV, D, S, ns = case
+    q, _, _, kq, vq = make_case(2, HQ, HKV, D, S, nbits, gs, seed=S + gs, outlier_frac=0.0)
+    out = fused_decode_attention(q, kq, vq, num_splits=ns)
+    assert_close_to_reference(out, oracle_attention_on_quant(q, kq, vq), str(case))
+
+
+@pytest.mark.parametrize("nbits,HQ,S", [(4, 8, 4127), (2, 8, 8263), (4, 12, 8251)])
+@pytest.mark.parametrize("append", [False, True])
+def test_short_rows_of_unaligned_blocks(nbits, HQ, S, append):
+    """Rows that end in the first chunk, just past it, and at the capacity."""
+    from tritonkv_amd.kernels import fused_decode_attention
+    from tritonkv_amd.quantize import append_kv
+
+    B, HKV, D, gs = 6, 2, 128, 32
+    q, k, v, kq, vq = make_case(B, HQ, HKV, D, S, nbits, gs, seed=S, outlier_frac=0.0)
+    lens = torch.tensor([1, 3, 31, 33, 290, S], dtype=torch.int32, device=DEV)
+    new = {}
+    want_k, want_v = kq.contiguous(), vq.contiguous()
+    if append:
+        g = torch.Generator().manual_seed(1)
+        kn, vn = (torch.randn(B, HKV, D, generator=g).to(torch.float16).to(DEV) for _ in range(2))
+        want_k, want_v = kq._map(torch.Tensor.clone), vq._map(torch.Tensor.clone)
+        append_kv(want_k, kn[:, :, None], lens - 1)
+        append_kv(want_v, vn[:, :, None], lens - 1)
+        new = dict(k_new=kn, v_new=vn)
+    out = fused_decode_attention(q, kq, vq, seq_lens=lens, num_splits=1, **new)
+    for got, want in ((kq, want_k), (vq, want_v)):
+        assert torch.equal(got.packed, want.packed)
+        assert torch.equal(got.scale.view(torch.int16), want.scale.view(torch.int16))
+    ref = oracle_attention_on_quant(q, want_k, want_v, seq_lens=lens.cpu().numpy())
+    assert_close_to_reference(out, ref, f"nbits={nbits} append={append}")

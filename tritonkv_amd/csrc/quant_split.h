@@ -609,8 +609,13 @@ quant_split_lds_kernel(SplitParams prm) {
       if constexpr (NG == 1) reinterpret_cast<uint32_t*>(ring + s * SG::BYTES + SG::ZERO_OFF)[i] = 0u;
     }
 
-  // Chunk k of this wave starts at token lo + 32 * (w + NW * k).
-  const int cb0 = lo + kChunk * w;
+  // Chunk k of this wave starts at token lo - head + 32 * (w + NW * k); the
+  // split's first chunk masks the `head` rows before lo (SplitParams::row_align).
+  constexpr bool kAlign = !PAGED && !KCH && VS == 1;
+  const int first = lo - (kAlign ? (int)(((uint32_t)unit * (uint32_t)prm.S + (uint32_t)lo) &
+                                         (uint32_t)prm.row_align)
+                                 : 0);
+  const int cb0 = first + kChunk * w;
   const int cstride = kChunk * NW;
   static_assert(NSTAGE >= 2 && (!PAGED || NSTAGE == 2), "ring depth");
   // Paged: page_next is the pool page of the chunk whose DMA is issued next;
@@ -811,7 +816,7 @@ quant_split_lds_kernel(SplitParams prm) {
   uint8_t* const patch = smem + NW * SM::WAVE;
   int cb_new = -1;  // first token of the chunk this wave patches, or -1
   int t_new = 0;    // the new token's row within that chunk
-  if (prm.k_new && L - 1 >= lo && L - 1 < hi && ((L - 1 - lo) / kChunk) % NW == w) {
+  if (prm.k_new && L - 1 >= lo && L - 1 < hi && ((L - 1 - first) / kChunk) % NW == w) {
     const int tn = L - 1;
     int64_t row = (int64_t)unit * prm.S + tn;
     bool use = true;
@@ -821,7 +826,7 @@ quant_split_lds_kernel(SplitParams prm) {
       row = ((int64_t)e * prm.HKV + hk) * prm.page_size + tn % prm.page_size;
     }
     if (use) {
-      cb_new = lo + kChunk * ((tn - lo) / kChunk);
+      cb_new = first + kChunk * ((tn - first) / kChunk);
       t_new = tn - cb_new;
       const int64_t xoff = (int64_t)unit * D * (prm.new_fp32 ? 4 : 2);
       float xk[KL::P], xv[VL::P];
@@ -862,6 +867,10 @@ quant_split_lds_kernel(SplitParams prm) {
   float zero_v = 0.0f;  // an opaque zero (see the one-group score fold)
   asm volatile("" : "+v"(zero_v));
   const float lscale = prm.qk_scale * __builtin_ldexpf(1.0f, 24 - eh);  // per lane (its head)
+
+  // A row before the split's start takes a score no key reaches.  It is
+  // finite, so a chunk whose other scores are all -inf keeps a finite maximum.
+  constexpr float x_head = -1e30f;
 
   // In the tail chunk, rows past the sequence hold whatever the cache holds
   // there (possibly NaN/Inf bit patterns in scale/zero): their V scale and
@@ -1018,6 +1027,12 @@ quant_split_lds_kernel(SplitParams prm) {
         }
         }  // NG > 1
       }
+      if constexpr (kAlign && SK == 0)  // the wave's first chunk is in stage 0
+        if (cb < lo) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (cb + tile_pt + 4 * j + i < lo) x[i] = x_head;
+        }
       if constexpr (TAIL) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -1194,6 +1209,14 @@ quant_split_lds_kernel(SplitParams prm) {
         }
       }
       }  // per-token key groups
+      if constexpr (kAlign && SK == 0)  // the wave's first chunk is in stage 0
+        if (cb < lo) {
+  #pragma unroll
+          for (int a = 0; a < 2; ++a)
+  #pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (cb + 16 * a + 4 * j + i < lo) x[4 * a + i] = x_head;
+        }
       if constexpr (TAIL) {
   #pragma unroll
         for (int a = 0; a < 2; ++a)
