@@ -119,12 +119,14 @@ SIGNATURES = {
 }
 
 _LIB = None
+_HOST = None
+_ADDRESSES: dict = {}
 _LOAD_ERROR: str | None = None
 
 
 def load():
     """Load the library (once).  Raises RuntimeError if it is absent or broken."""
-    global _LIB, _LOAD_ERROR
+    global _LIB, _HOST, _LOAD_ERROR
     if _LIB is not None:
         return _LIB
     if not os.path.exists(LIB_PATH):
@@ -140,8 +142,21 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = restype
+    try:
+        from . import _hostcall
+    except ImportError as exc:
+        _LOAD_ERROR = f"tritonkv_amd/_hostcall.so: {exc}; run `python -m tritonkv_amd.build`"
+        raise RuntimeError(_LOAD_ERROR) from exc
+    _HOST = _hostcall
     _LIB = lib
     return lib
+
+
+def host():
+    """The CPython module of repeated calls (``csrc/host_call.cpp``)."""
+    if _HOST is None:
+        load()
+    return _HOST
 
 
 def load_error() -> str | None:
@@ -168,6 +183,23 @@ def check(rc: int, what: str) -> None:
 
 def stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def address(name: str) -> int:
+    """Address of a library entry point."""
+    if name not in _ADDRESSES:
+        _ADDRESSES[name] = ctypes.cast(getattr(load(), name), ctypes.c_void_p).value
+    return _ADDRESSES[name]
+
+
+def launch(device: torch.device, name: str, *args) -> int:
+    """The status of library call ``name`` with ``args`` on the device's current stream."""
+    fn = getattr(load(), name)
+    stream = _HOST.raw_stream(device.index)
+    if stream is not None:
+        return fn(*args, stream)
+    with torch.cuda.device(device):
+        return fn(*args, stream_handle(device))
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -5,7 +5,8 @@
 Each ``.hip`` source is compiled to an object in parallel (the quantized split
 kernel's instantiations are spread over one file per K/V bit-width pair and
 head-column width), then
-linked into ``tritonkv_amd/libtkv_hip.so``.  Flags:
+linked into ``tritonkv_amd/libtkv_hip.so``.  ``host_call.cpp`` (host code, against
+the installed torch) becomes ``tritonkv_amd/_hostcall.so``.  Flags:
 
 * ``--offload-arch=gfx950`` only -- no other targets, no host fallback;
 * ``-O3`` without fast-math: the quantizer needs IEEE binary32 division and
@@ -38,6 +39,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libtkv_hip.so")
+HOSTCALL = os.path.join(PKG, "_hostcall.so")
 SOURCES = ["decode_attention.hip", "quant_pack.hip", "dequant.hip", "runtime.hip"] + [
     f"quant_split_{bits}{hc}.hip" for bits in ("k4v4", "k2v2", "k4v2", "k2v4") for hc in ("", "_h4", "_h8")]
 ARCH = "gfx950"
@@ -73,11 +75,36 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_hostcall() -> str:
+    """The CPython module of repeated decode calls (host code only), against the
+    installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [f for d in (*cpp_extension.include_paths(), "/opt/rocm/include",
+                       sysconfig.get_paths()["include"]) for f in ("-isystem", d)]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOSTCALL + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
+           os.path.join(CSRC, "host_call.cpp"), "-o", tmp, f"-L{lib}", "-lc10", "-lc10_hip",
+           "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for host_call.cpp:\n{res.stderr[-6000:]}")
+    os.replace(tmp, HOSTCALL)
+    return HOSTCALL
+
+
 def build(verbose: bool = False) -> str:
     """Compile every HIP source for gfx950 and link the shared library."""
     os.makedirs(OBJ, exist_ok=True)
-    with cf.ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with cf.ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as ex:
+        host = ex.submit(build_hostcall)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)

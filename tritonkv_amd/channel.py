@@ -32,8 +32,8 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .kernels.fused_decode_attn import (_aligned16, _cache_arg, _check_out, _seq_lens_arg, _workspace_for,
-                                        choose_waves, plan_splits, triton_available)
+from .kernels.fused_decode_attn import (_aligned16, _backend, _cache_arg, _check_out, _keep_call, _prepared,
+                                        _seq_lens_arg, _workspace_for, choose_waves, plan_splits)
 from .quantize import QuantizedTensor, _check_bits, _require_gpu, append_kv, empty_cache
 
 BLOCK = 32  # tokens per key block
@@ -104,12 +104,11 @@ def append_keys_per_channel(ck: ChannelQuantizedKeys, k_new: torch.Tensor,
                                   or positions.device != k_new.device):
         raise ValueError("positions must be an int32 tensor of B entries on the cache's device")
     kc = k_new.contiguous()
-    with torch.cuda.device(k_new.device):
-        rc = _lib.load().tkv_quantize_keys_channel(
-            kc.data_ptr(), int(kc.dtype == torch.float32), B, HKV, N, D, ck.nbits,
-            _lib.ptr(positions), S, ck.packed.data_ptr(), ck.scale.data_ptr(),
-            ck.zero.data_ptr(), _lib.stream_handle(k_new.device))
-        _lib.check(rc, "append_keys_per_channel")
+    rc = _lib.launch(k_new.device, "tkv_quantize_keys_channel",
+                     kc.data_ptr(), int(kc.dtype == torch.float32), B, HKV, N, D, ck.nbits,
+                     _lib.ptr(positions), S, ck.packed.data_ptr(), ck.scale.data_ptr(),
+                     ck.zero.data_ptr())
+    _lib.check(rc, "append_keys_per_channel")
     return ck
 
 
@@ -151,6 +150,16 @@ def channel_decode_attention(
     ``q_lens`` is the same, so the split plan of a batch without lengths
     applies.
     """
+    key = None
+    if _workspace is not None:
+        key = ("channel", ck.nbits, ck.head_dim, vq.nbits, vq.group_size, vq.head_dim, sm_scale,
+               block_n, num_splits, equal_lengths)
+        prep = _prepared(_workspace, key)
+        if prep is not None:
+            res = prep.run(out, q, ck.packed, ck.scale, ck.zero, vq.packed, vq.scale, vq.zero,
+                           k_res, v_res, res_lens, q_lens, None, None)
+            if res is not None:
+                return res
     for t, what in ((q, "q"), (k_res, "k_res"), (v_res, "v_res")):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{what} must be a tensor")
@@ -171,7 +180,7 @@ def channel_decode_attention(
     R = k_res.shape[2]
     qlens = _seq_lens_arg(q_lens, B, S, q.device)
     rlens = _seq_lens_arg(res_lens, B, R, q.device)
-    ok, why = triton_available()
+    ok, why = _backend(q)
     if not ok:
         raise RuntimeError(f"channel_decode_attention requires the tritonkv_amd HIP backend: {why}")
 
@@ -179,6 +188,7 @@ def channel_decode_attention(
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group,
                                             ragged=q_lens is not None and not equal_lengths)
+    q_in = q
     if q.dtype not in (torch.float16, torch.float32):
         q = q.float()
     q = _aligned16(q)
@@ -187,7 +197,7 @@ def channel_decode_attention(
     ks, kz, vs, vz = (_cache_arg(t, 4, n) for t, n in ((ck.scale, "ck.scale"), (ck.zero, "ck.zero"),
                                                        (vq.scale, "vq.scale"), (vq.zero, "vq.zero")))
     out = _check_out(out, B, HQ, D, q.device)
-    acc, maxs, sums, _ = _workspace_for(_workspace, B, HQ, num_splits + 1, D, q.device, HKV)
+    acc, maxs, sums, counters = _workspace_for(_workspace, B, HQ, num_splits + 1, D, q.device, HKV)
     args = _lib.DecodeArgs(
         q=q.data_ptr(), q_is_fp32=int(q.dtype == torch.float32),
         k=kp.data_ptr(), k_scale=ks.data_ptr(), k_zero=kz.data_ptr(),
@@ -198,10 +208,15 @@ def channel_decode_attention(
         split_size=split_size, num_splits=num_splits, counters=None,
         waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, k_nbits=ck.nbits,
                            v_nbits=vq.nbits, group_size=vq.group_size), key_block=BLOCK)
-    with torch.cuda.device(q.device):
-        rc = _lib.load().tkv_channel_decode_attention(
-            args, kr.data_ptr(), vr.data_ptr(), _lib.ptr(rlens), R, _lib.stream_handle(q.device))
+    rc = _lib.launch(q.device, "tkv_channel_decode_attention", args, kr.data_ptr(), vr.data_ptr(),
+                     _lib.ptr(rlens), R)
     _lib.check(rc, "channel_decode_attention")
+    if key is not None and q is q_in:
+        _keep_call(_workspace, key, args, "tkv_channel_decode_attention",
+                   "channel_decode_attention", out, (acc, maxs, sums, counters), q,
+                   (ck.packed, ck.scale, ck.zero, vq.packed, vq.scale, vq.zero, k_res, v_res,
+                    res_lens), q_lens,
+                   window=(kr.data_ptr(), vr.data_ptr(), _lib.ptr(rlens), R))
     return out
 
 
@@ -322,15 +337,14 @@ class ChannelKVCache:
         v, vs = _strided_rows(v)
         B, HKV, N, D = k.shape
         kc, vc = self.keys, self.values
-        with torch.cuda.device(self.k_res.device):
-            rc = _lib.load().tkv_channel_extend(
-                k.data_ptr(), ks, v.data_ptr(), vs, B, HKV, N, D, kc.nbits, vc.nbits,
-                vc.group_size, self.quantized, self.k_res.data_ptr(), self.v_res.data_ptr(), BLOCK,
-                self._qlens.data_ptr(), self._rlens.data_ptr(), self.capacity,
-                kc.packed.data_ptr(), kc.scale.data_ptr(), kc.zero.data_ptr(),
-                vc.packed.data_ptr(), vc.scale.data_ptr(), vc.zero.data_ptr(),
-                _lib.stream_handle(self.k_res.device))
-            _lib.check(rc, "ChannelKVCache.extend")
+        rc = _lib.launch(
+            self.k_res.device, "tkv_channel_extend",
+            k.data_ptr(), ks, v.data_ptr(), vs, B, HKV, N, D, kc.nbits, vc.nbits,
+            vc.group_size, self.quantized, self.k_res.data_ptr(), self.v_res.data_ptr(), BLOCK,
+            self._qlens.data_ptr(), self._rlens.data_ptr(), self.capacity,
+            kc.packed.data_ptr(), kc.scale.data_ptr(), kc.zero.data_ptr(),
+            vc.packed.data_ptr(), vc.scale.data_ptr(), vc.zero.data_ptr())
+        _lib.check(rc, "ChannelKVCache.extend")
         self.quantized += N // BLOCK * BLOCK
         self.window = N % BLOCK
 
@@ -356,21 +370,19 @@ class ChannelKVCache:
         B, HKV, _, D = self.k_res.shape
         kk = k.to(torch.float16).contiguous()
         vv = v.to(torch.float16).contiguous()
-        lib, st = _lib.load(), _lib.stream_handle(self.k_res.device)
-        with torch.cuda.device(self.k_res.device):
-            rc = lib.tkv_channel_window_append(kk.data_ptr(), vv.data_ptr(), B, HKV, D,
-                                               self.k_res.data_ptr(), self.v_res.data_ptr(), BLOCK,
-                                               self._rlens.data_ptr(), st)
-            _lib.check(rc, "ChannelKVCache.step (window append)")
+        dev = self.k_res.device
+        rc = _lib.launch(dev, "tkv_channel_window_append", kk.data_ptr(), vv.data_ptr(), B, HKV, D,
+                         self.k_res.data_ptr(), self.v_res.data_ptr(), BLOCK, self._rlens.data_ptr())
+        _lib.check(rc, "ChannelKVCache.step (window append)")
         out = self.attend(q, sm_scale=sm_scale, out=out)
         ks, vs = self.keys, self.values
-        with torch.cuda.device(self.k_res.device):
-            rc = lib.tkv_channel_window_flush(
-                self.k_res.data_ptr(), self.v_res.data_ptr(), B, HKV, D, ks.nbits, vs.nbits,
-                vs.group_size, BLOCK, self._qlens.data_ptr(), self._rlens.data_ptr(),
-                self.capacity, ks.packed.data_ptr(), ks.scale.data_ptr(), ks.zero.data_ptr(),
-                vs.packed.data_ptr(), vs.scale.data_ptr(), vs.zero.data_ptr(), st)
-            _lib.check(rc, "ChannelKVCache.step (window flush)")
+        rc = _lib.launch(
+            dev, "tkv_channel_window_flush",
+            self.k_res.data_ptr(), self.v_res.data_ptr(), B, HKV, D, ks.nbits, vs.nbits,
+            vs.group_size, BLOCK, self._qlens.data_ptr(), self._rlens.data_ptr(),
+            self.capacity, ks.packed.data_ptr(), ks.scale.data_ptr(), ks.zero.data_ptr(),
+            vs.packed.data_ptr(), vs.scale.data_ptr(), vs.zero.data_ptr())
+        _lib.check(rc, "ChannelKVCache.step (window flush)")
         self.window += 1
         if self.window == BLOCK:
             self.quantized += BLOCK

@@ -28,16 +28,15 @@ from .. import _lib
 from .fused_decode_attn import (
     TOKENS_PER_WORKGROUP_FP16,
     _aligned16,
+    _backend,
     _cache_arg,
     _check_out,
-    _PreparedCall,
+    _keep_call,
     _prepared,
     _seq_lens_arg,
-    _tensor_key,
     _workspace_for,
     choose_waves,
     plan_splits,
-    triton_available,
 )
 
 
@@ -64,12 +63,10 @@ def fp16_decode_attention(
     """
     key = None
     if _workspace is not None:
-        key = ("fp16", q.shape, q.dtype, q.device, q.is_contiguous(), _tensor_key(k),
-               _tensor_key(v), sm_scale, block_n, num_splits, _tensor_key(out),
-               _tensor_key(seq_lens), equal_lengths)
+        key = ("fp16", sm_scale, block_n, num_splits, equal_lengths)
         prep = _prepared(_workspace, key)
         if prep is not None:
-            res = prep.run(q, out)
+            res = prep.run(out, q, k, v, seq_lens, None, None)
             if res is not None:
                 return res
     B, HQ, D = q.shape
@@ -81,7 +78,7 @@ def fp16_decode_attention(
     if k.device != q.device or v.device != q.device:
         raise ValueError("q, k and v must be on the same device")
 
-    ok, why = triton_available()
+    ok, why = _backend(q)
     if not ok:
         raise RuntimeError(f"tritonkv_amd HIP backend unavailable: {why}")
 
@@ -109,11 +106,10 @@ def fp16_decode_attention(
         B=B, HQ=HQ, HKV=HKV, S=S, D=D, k_nbits=16, v_nbits=16, group_size=D,
         sm_scale=float(sm_scale), split_size=split_size, num_splits=num_splits,
         counters=None, waves=choose_waves(B, HKV, group, split_size, num_splits))
-    with torch.cuda.device(q.device):
-        rc = _lib.load().tkv_fp16_decode_attention(args, _lib.stream_handle(q.device))
+    rc = _lib.launch(q.device, "tkv_fp16_decode_attention", args)
     _lib.check(rc, "fp16_decode_attention")
     # k / v are read in place; a converted copy (not fp16, not contiguous) is not kept
     if key is not None and q is q_in and k is k_in and v is v_in:
-        _workspace["call"] = _PreparedCall(key, args, _lib.load().tkv_fp16_decode_attention,
-                                           "fp16_decode_attention", (B, HQ, D), q.device, False)
+        _keep_call(_workspace, key, args, "tkv_fp16_decode_attention", "fp16_decode_attention",
+                   out, (acc, maxs, sums), q, (k, v), seq_lens)
     return out

@@ -68,6 +68,12 @@ def triton_available() -> tuple[bool, str]:
 hip_available = triton_available
 
 
+def _backend(t: torch.Tensor) -> tuple[bool, str]:
+    """:func:`triton_available`, without asking the runtime again for a tensor
+    that is on the GPU already."""
+    return (True, "") if t.is_cuda and _lib.load_error() is None else triton_available()
+
+
 def _next_pow2(x: int) -> int:
     return 1 << (x - 1).bit_length()
 
@@ -367,40 +373,50 @@ def _new_key(t):
 
 
 class _PreparedCall:
-    """The validated argument block of a decode call, kept in the caller's
-    ``_workspace`` under ``"call"``.  A later call whose key matches (same
-    caches, buffers, shapes and flags; q and the new token's rows may be new
-    tensors of the same shape) reuses it: only those pointers are refreshed.
-    This takes validation, the split plan and the construction of the ctypes
-    argument block (most of the ~16-20 us an eager call spent on the host)
-    off every step of a decode loop."""
+    """A checked decode call, kept in the caller's ``_workspace`` under ``"call"``.
+    ``key`` holds the options it was planned with; the forms of its tensors
+    (and the argument block) live in the native call object, which compares
+    every tensor of a later call with them (storage, shape, dtype, device,
+    layout) and launches: q, the new token's rows and the output may be new
+    tensors of the same form.  This takes validation, the split plan and the
+    construction of the ctypes argument block off every step of a decode loop."""
 
-    __slots__ = ("key", "args", "entry", "what", "out_shape", "device", "new")
+    __slots__ = ("key", "call", "what", "out_shape", "device", "buffers")
 
-    def __init__(self, key, args, entry, what, out_shape, device, new):
-        self.key, self.args, self.entry, self.what = key, args, entry, what
-        self.out_shape, self.device, self.new = out_shape, device, new
+    def __init__(self, key, call, what, out_shape, device, buffers):
+        self.key, self.call, self.what = key, call, what
+        self.out_shape, self.device = out_shape, device
+        self.buffers = buffers  # the argument block points into them
 
-    def run(self, q, out, k_new=None, v_new=None):
-        """Launch with this q (and new token); None when q does not qualify
-        (misaligned), so that the caller takes the full path."""
-        qp = q.data_ptr()
-        if qp % 16:
-            return None
-        a = self.args
-        a.q = qp
-        if self.new:
-            a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
+    def run(self, out, *tensors):
+        """Launch with these tensors; None (nothing launched) when one does not
+        have its checked form, so that the caller takes the full path."""
         if out is None:
             out = torch.empty(self.out_shape, device=self.device, dtype=torch.float32)
-            a.out = out.data_ptr()
-        if self.device.index == torch.cuda.current_device():
-            rc = self.entry(a, torch.cuda.current_stream().cuda_stream)
-        else:
-            with torch.cuda.device(self.device):
-                rc = self.entry(a, torch.cuda.current_stream().cuda_stream)
-        _lib.check(rc, self.what)
+        rc = _lib.host().run(self.call, out, *tensors)
+        if rc is None:
+            return None
+        if rc:
+            _lib.check(rc, self.what)
         return out
+
+
+_OUT_OFFSET, _Q_OFFSET, _K_NEW_OFFSET, _V_NEW_OFFSET = (
+    getattr(_lib.DecodeArgs, f).offset for f in ("out", "q", "k_new", "v_new"))
+
+
+def _keep_call(ws, key, args, entry, what, out, buffers, q, caches, lens, new=(None, None),
+               window=None):
+    """Put a call that just ran into the workspace for reuse, if every tensor
+    was used as it was passed (contiguous, plain storage)."""
+    keys = (_tensor_key(q), _tensor_key(lens), _new_key(new[0]), _new_key(new[1]))
+    if not all(k is None or k[-1] for k in keys):  # the caches: prepare() looks
+        return
+    slots = ((out, _OUT_OFFSET, 16), (q, _Q_OFFSET, 16), *((t, -1, 1) for t in caches),
+             (lens, -1, 1), (new[0], _K_NEW_OFFSET, 1), (new[1], _V_NEW_OFFSET, 1))
+    call = _lib.host().prepare(bytes(args), _lib.address(entry), out.device.index, slots, window)
+    if call is not None:
+        ws["call"] = _PreparedCall(key, call, what, tuple(out.shape), out.device, buffers)
 
 
 def _prepared(ws, key):
@@ -448,16 +464,13 @@ def fused_decode_attention(
     """
     key = None
     if _workspace is not None:
-        key = ("fused", q.shape, q.dtype, q.device, q.is_contiguous(),
-               _tensor_key(kq.packed), _tensor_key(kq.scale), _tensor_key(kq.zero),
-               _tensor_key(vq.packed), _tensor_key(vq.scale), _tensor_key(vq.zero),
-               kq.nbits, vq.nbits, kq.group_size, vq.group_size, kq.head_dim, vq.head_dim,
-               sm_scale, block_n, num_splits, fold_zp, _tensor_key(out), _tensor_key(seq_lens),
-               allow_mixed_bits, fused_combine, _new_key(k_new), _new_key(v_new),
-               dispatch_order, equal_lengths)
+        key = ("fused", kq.nbits, vq.nbits, kq.group_size, vq.group_size, kq.head_dim,
+               vq.head_dim, sm_scale, block_n, num_splits, fold_zp, allow_mixed_bits,
+               fused_combine, dispatch_order, equal_lengths)
         prep = _prepared(_workspace, key)
         if prep is not None:
-            res = prep.run(q, out, k_new, v_new)
+            res = prep.run(out, q, kq.packed, kq.scale, kq.zero, vq.packed, vq.scale, vq.zero,
+                           seq_lens, k_new, v_new)
             if res is not None:
                 return res
     if kq.group_size != vq.group_size or (kq.nbits != vq.nbits and not allow_mixed_bits):
@@ -488,7 +501,7 @@ def fused_decode_attention(
                                                           (vq.scale, "vq.scale"),
                                                           (vq.zero, "vq.zero")))
 
-    ok, why = triton_available()
+    ok, why = _backend(q)
     if not ok:
         raise RuntimeError(f"fused_decode_attention requires the tritonkv_amd HIP backend: {why}")
 
@@ -520,14 +533,11 @@ def fused_decode_attention(
                            v_nbits=vq.nbits, group_size=kq.group_size),
         k_new=_lib.ptr(kn), v_new=_lib.ptr(vn), new_is_fp32=new_f32,
         work_order=_lib.ptr(order))
-    with torch.cuda.device(q.device):
-        rc = _lib.load().tkv_fused_decode_attention(args, _lib.stream_handle(q.device))
+    rc = _lib.launch(q.device, "tkv_fused_decode_attention", args)
     _lib.check(rc, "fused_decode_attention")
-    # q is kept as given unless it had to be converted or realigned (then no reuse)
-    if key is not None and q is q_in and kp is kq.packed and vp is vq.packed and \
-            ks is kq.scale and kz is kq.zero and vs is vq.scale and vz is vq.zero:
-        _workspace["call"] = _PreparedCall(key, args, _lib.load().tkv_fused_decode_attention,
-                                           "fused_decode_attention", (B, HQ, D), q.device,
-                                           kn is not None)
+    if key is not None and q is q_in:  # q as given, not converted or realigned
+        _keep_call(_workspace, key, args, "tkv_fused_decode_attention", "fused_decode_attention",
+                   out, (acc, maxs, sums, counters, order), q,
+                   (kq.packed, kq.scale, kq.zero, vq.packed, vq.scale, vq.zero), seq_lens,
+                   (k_new, v_new))
     return out
-

@@ -29,9 +29,8 @@ import math
 import torch
 
 from . import _lib
-from .kernels.fused_decode_attn import (_aligned16, _check_out, _order_for, _workspace_for,
-                                        choose_waves, new_token_args, plan_splits,
-                                        triton_available)
+from .kernels.fused_decode_attn import (_aligned16, _backend, _check_out, _keep_call, _order_for,
+                                        _prepared, _workspace_for, choose_waves, new_token_args, plan_splits)
 from .quantize import QuantizedTensor, _check_bits, _require_gpu, empty_cache
 
 PAGE_MULTIPLE = 32
@@ -96,13 +95,13 @@ def paged_append(pool: QuantizedTensor, x_new: torch.Tensor, block_table: torch.
         raise ValueError("positions must be an int32 tensor of B entries on the pool's device")
     table = _check_table(block_table, B, x_new.device)
     xc = x_new.contiguous()
-    with torch.cuda.device(x_new.device):
-        rc = _lib.load().tkv_paged_quantize_pack(
-            xc.data_ptr(), int(xc.dtype == torch.float32), B, HKV, N, D, pool.nbits,
-            pool.group_size, positions.contiguous().data_ptr(), table.data_ptr(),
-            table.shape[1], page_size, num_pages, pool.packed.data_ptr(), pool.scale.data_ptr(),
-            pool.zero.data_ptr(), _lib.stream_handle(x_new.device))
-        _lib.check(rc, "paged_append")
+    rc = _lib.launch(
+        x_new.device, "tkv_paged_quantize_pack",
+        xc.data_ptr(), int(xc.dtype == torch.float32), B, HKV, N, D, pool.nbits,
+        pool.group_size, positions.contiguous().data_ptr(), table.data_ptr(),
+        table.shape[1], page_size, num_pages, pool.packed.data_ptr(), pool.scale.data_ptr(),
+        pool.zero.data_ptr())
+    _lib.check(rc, "paged_append")
     return pool
 
 
@@ -136,8 +135,19 @@ def paged_decode_attention(
     ``v_new`` fuse the step's append into the same launch (the token lands at
     ``seq_lens[b] - 1``), bit-identical to :func:`paged_append` followed by
     this call.  ``dispatch_order`` and ``equal_lengths`` as for
-    ``fused_decode_attention``.
+    ``fused_decode_attention``, as is the reuse of a workspace's checked call.
     """
+    key = None
+    if _workspace is not None:
+        key = ("paged", k_pool.nbits, v_pool.nbits, k_pool.group_size, v_pool.group_size,
+               k_pool.head_dim, v_pool.head_dim, sm_scale, block_n, num_splits, allow_mixed_bits,
+               dispatch_order, equal_lengths)
+        prep = _prepared(_workspace, key)
+        if prep is not None:
+            res = prep.run(out, q, k_pool.packed, k_pool.scale, k_pool.zero, v_pool.packed,
+                           v_pool.scale, v_pool.zero, block_table, seq_lens, k_new, v_new)
+            if res is not None:
+                return res
     if k_pool.group_size != v_pool.group_size or (k_pool.nbits != v_pool.nbits
                                                   and not allow_mixed_bits):
         raise ValueError("K and V must use the same nbits/group_size")
@@ -162,7 +172,7 @@ def paged_decode_attention(
     if q.device != k_pool.device or v_pool.device != k_pool.device:
         raise ValueError("q and the pools must be on the same device")
     kn, vn, new_f32 = new_token_args(k_new, v_new, B, HKV, D, q.device)
-    ok, why = triton_available()
+    ok, why = _backend(q)
     if not ok:
         raise RuntimeError(f"paged_decode_attention requires the tritonkv_amd HIP backend: {why}")
 
@@ -170,11 +180,12 @@ def paged_decode_attention(
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     ragged = seq_lens is not None and not equal_lengths
     _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged)
+    q_in = q
     if q.dtype not in (torch.float16, torch.float32):
         q = q.float()
     q = _aligned16(q)
     out = _check_out(out, B, HQ, D, q.device)
-    acc, maxs, sums, _ = _workspace_for(_workspace, B, HQ, num_splits, D, q.device, HKV)
+    acc, maxs, sums, counters = _workspace_for(_workspace, B, HQ, num_splits, D, q.device, HKV)
     lens = seq_lens.contiguous() if seq_lens is not None else None
     order = _order_for(_workspace, B, HKV, num_splits, q.device, seq_lens if ragged else None,
                        dispatch_order, group, D)
@@ -192,9 +203,13 @@ def paged_decode_attention(
         block_table=table.data_ptr(), block_table_stride=table.shape[1], page_size=page_size,
         num_pages=num_pages, k_new=_lib.ptr(kn), v_new=_lib.ptr(vn), new_is_fp32=new_f32,
         work_order=_lib.ptr(order))
-    with torch.cuda.device(q.device):
-        rc = _lib.load().tkv_fused_decode_attention(args, _lib.stream_handle(q.device))
+    rc = _lib.launch(q.device, "tkv_fused_decode_attention", args)
     _lib.check(rc, "paged_decode_attention")
+    if key is not None and q is q_in:
+        _keep_call(_workspace, key, args, "tkv_fused_decode_attention", "paged_decode_attention",
+                   out, (acc, maxs, sums, counters, order), q,
+                   (k_pool.packed, k_pool.scale, k_pool.zero, v_pool.packed, v_pool.scale,
+                    v_pool.zero, block_table), seq_lens, (k_new, v_new))
     return out
 
 
