@@ -258,7 +258,7 @@ int tkv_quantize_keys_channel(const void *x, int32_t x_is_fp32, int32_t B, int32
  * 32-token blocks of the N tokens are quantized into the history at token
  * `start` (a multiple of 32; start + N <= S_cap) -- keys exactly as
  * tkv_quantize_keys_channel, values as tkv_quantize_pack -- the rest goes to window rows 0 .., and every row's q_lens becomes
- * start + whole blocks, its res_lens the rest.  Three launches.  No
+ * start + whole blocks, its res_lens the rest.  Two launches.  No
  * counterpart in the reference (it plans the format). */
 int tkv_channel_extend(const void *k, const int64_t *k_strides, const void *v,
                        const int64_t *v_strides, int32_t B, int32_t HKV, int32_t N, int32_t D,

@@ -306,7 +306,7 @@ class ChannelKVCache:
 
     def extend(self, k: torch.Tensor, v: torch.Tensor) -> None:
         """Append ``(B, HKV, N, D)`` keys and values from the host (prefill).
-        With an empty window that is three launches, which read ``k`` and ``v``
+        With an empty window that is two launches, which read ``k`` and ``v``
         in the layout they have (rows contiguous, strides 16-byte multiples)."""
         self._check_tokens(k, v)
         if k.dtype != torch.float16:

@@ -520,56 +520,78 @@ struct KeyBlock {
   }
 };
 
-// A block whose destination does not start on a 32-token boundary, or does not
-// fit [0, S_cap), is not written.  Blocks of a batch row are dealt to waves
-// heads first for a token-major source (neighbouring waves then read
-// neighbouring memory), tokens first otherwise.
+// Workgroup wg's four waves of the key blocks of batch row b.  A block whose
+// destination does not start on a 32-token boundary, or does not fit
+// [0, S_cap), is not written.  Blocks are dealt to waves heads first for a
+// token-major source (neighbouring waves then read neighbouring memory), tokens
+// first otherwise.
 template <int D, int NB, bool F32>
-__global__ void __launch_bounds__(256)
-quantize_keys_channel_kernel(TokenSource src, bool wide, int B, int HKV, int NBLK,
-                             const int32_t* __restrict__ positions, int start, int S_cap,
-                             uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
-                             uint16_t* __restrict__ zero) {
+__device__ __forceinline__ void quantize_key_blocks(const TokenSource& src, bool wide, int wg, int b,
+                                                    int HKV, int NBLK, int64_t start, int S_cap,
+                                                    uint8_t* __restrict__ packed,
+                                                    uint16_t* __restrict__ scale,
+                                                    uint16_t* __restrict__ zero) {
   using K = KeyBlock<D, NB, F32>;
   constexpr int T = K::T;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int first = ((int)blockIdx.x * 4 + w) * K::BPW, blocks = HKV * NBLK;
+  const int first = (wg * 4 + w) * K::BPW, blocks = HKV * NBLK;
   if (first >= blocks) return;  // whole wave
   const int i = first + (K::BPW > 1 ? lane / K::LB : 0);
   const int ii = min(i, blocks - 1);
   const bool heads_first = src.st != D;
   const int q = ii / (heads_first ? HKV : NBLK), m = ii - q * (heads_first ? HKV : NBLK);
   const int kv = heads_first ? m : q, tb = heads_first ? q : m;
-  for (int b = blockIdx.y; b < B; b += gridDim.y) {
-    const int64_t off = b * src.sb + kv * src.sh + (int64_t)tb * T * src.st;
-    const int64_t dst_t = (int64_t)(positions ? positions[b] : start) + (int64_t)tb * T;
-    const bool ok = i < blocks && dst_t >= 0 && dst_t % T == 0 && dst_t + T <= S_cap;
-    const int64_t bh = (int64_t)b * HKV + kv;
-    const int64_t meta = ok ? (bh * (S_cap / T) + dst_t / T) * D : 0;
-    K::quantize(F32 ? (const void*)(static_cast<const float*>(src.x) + off)
-                    : (const void*)(static_cast<const uint16_t*>(src.x) + off),
-                src.st, wide, lane, ok, packed + (ok ? (bh * S_cap + dst_t) * K::DP : 0),
-                scale + meta, zero + meta);
-  }
+  const int64_t off = b * src.sb + kv * src.sh + (int64_t)tb * T * src.st;
+  const int64_t dst_t = start + (int64_t)tb * T;
+  const bool ok = i < blocks && dst_t >= 0 && dst_t % T == 0 && dst_t + T <= S_cap;
+  const int64_t bh = (int64_t)b * HKV + kv;
+  const int64_t meta = ok ? (bh * (S_cap / T) + dst_t / T) * D : 0;
+  K::quantize(F32 ? (const void*)(static_cast<const float*>(src.x) + off)
+                  : (const void*)(static_cast<const uint16_t*>(src.x) + off),
+              src.st, wide, lane, ok, packed + (ok ? (bh * S_cap + dst_t) * K::DP : 0), scale + meta,
+              zero + meta);
 }
 
-// The tokens of a prompt past its last whole block into the window, rows
-// [0, rest) of every (b, kv head), and the batch row's lengths.
+template <int D, int NB, bool F32>
 __global__ void __launch_bounds__(256)
-channel_tail_kernel(TokenSource ks, TokenSource vs, int rest, int D, uint16_t* __restrict__ k_res,
-                    uint16_t* __restrict__ v_res, int32_t* __restrict__ q_lens,
-                    int32_t* __restrict__ res_lens, int q_len) {
+quantize_keys_channel_kernel(TokenSource src, bool wide, int B, int HKV, int NBLK,
+                             const int32_t* __restrict__ positions, int S_cap,
+                             uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
+                             uint16_t* __restrict__ zero) {
+  for (int b = blockIdx.y; b < B; b += gridDim.y)
+    quantize_key_blocks<D, NB, F32>(src, wide, blockIdx.x, b, HKV, NBLK, positions ? positions[b] : 0,
+                                    S_cap, packed, scale, zero);
+}
+
+// A prompt's keys and what lies past its last whole block, in one launch:
+// workgroups x < key_wgs quantize key blocks to token `start` on; workgroup
+// key_wgs + kv copies the last `rest` tokens of kv head kv into rows
+// [0, rest) of the windows (their own launch took 3-5 us behind the values'),
+// and the first of them sets the batch row's lengths.
+template <int D, int NB>
+__global__ void __launch_bounds__(256)
+channel_extend_kernel(TokenSource ks, TokenSource vs, int key_wgs, int HKV, int NBLK, int start,
+                      int S_cap, uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
+                      uint16_t* __restrict__ zero, int rest, uint16_t* __restrict__ k_res,
+                      uint16_t* __restrict__ v_res, int32_t* __restrict__ q_lens,
+                      int32_t* __restrict__ res_lens) {
   constexpr int T = 32;
-  const int kv = blockIdx.x, b = blockIdx.y, n = rest * D / 8;  // 16-byte vectors per tensor
+  const int b = blockIdx.y;
+  if ((int)blockIdx.x < key_wgs) {
+    quantize_key_blocks<D, NB, false>(ks, true, blockIdx.x, b, HKV, NBLK, start, S_cap, packed, scale, zero);
+    return;
+  }
+  const int kv = blockIdx.x - key_wgs, n = rest * D / 8;  // 16-byte vectors per tensor
   for (int i = threadIdx.x; i < 2 * n; i += blockDim.x) {
     const TokenSource& s = i < n ? ks : vs;
     const int e = (i < n ? i : i - n) * 8, t = e / D, d = e % D;
-    const uint16_t* from = static_cast<const uint16_t*>(s.x) + b * s.sb + kv * s.sh + t * s.st + d;
-    uint16_t* to = (i < n ? k_res : v_res) + (((int64_t)b * gridDim.x + kv) * T + t) * D + d;
+    const uint16_t* from =
+        static_cast<const uint16_t*>(s.x) + b * s.sb + kv * s.sh + (int64_t)(NBLK * T + t) * s.st + d;
+    uint16_t* to = (i < n ? k_res : v_res) + (((int64_t)b * HKV + kv) * T + t) * D + d;
     *reinterpret_cast<u4*>(to) = *reinterpret_cast<const u4*>(from);
   }
   if (kv == 0 && threadIdx.x == 0) {
-    q_lens[b] = q_len;
+    q_lens[b] = start + NBLK * T;
     res_lens[b] = rest;
   }
 }
@@ -844,36 +866,33 @@ static void launch_quantize(const TokenSource& src, bool f32, int B, int HKV, in
   }
 }
 
-template <int D, int NB, bool F32>
-static void launch_key_blocks(const TokenSource& src, int B, int HKV, int nblk, const int32_t* pos,
-                              int start, int S_cap, uint8_t* pk, uint16_t* sc, uint16_t* zr,
-                              hipStream_t st) {
-  constexpr int per_wg = 4 * KeyBlock<D, NB, F32>::BPW;
-  constexpr int pair = F32 ? 8 : 4;  // bytes of a lane's two channels
-  const uintptr_t align = (uintptr_t)src.x | (uintptr_t)(src.sb * pair / 2) |
-                          (uintptr_t)(src.sh * pair / 2) | (uintptr_t)(src.st * pair / 2);
-  const dim3 grid((unsigned)(((int64_t)HKV * nblk + per_wg - 1) / per_wg), (unsigned)(B < 65535 ? B : 65535));
-  quantize_keys_channel_kernel<D, NB, F32><<<grid, 256, 0, st>>>(
-      src, !(align & (pair - 1)), B, HKV, nblk, pos, start, S_cap, pk, sc, zr);
+// Workgroups of four waves for the nblk key blocks of HKV heads.
+template <int D>
+static unsigned key_workgroups(int HKV, int nblk) {
+  constexpr int per_wg = 4 * KeyBlock<D, 4, false>::BPW;
+  return (unsigned)(((int64_t)HKV * nblk + per_wg - 1) / per_wg);
 }
 
-static int launch_keys_channel(const TokenSource& src, bool f32, int B, int HKV, int nblk, int D,
-                               int nbits, const int32_t* pos, int start, int S_cap, uint8_t* pk,
-                               uint16_t* sc, uint16_t* zr, hipStream_t st) {
-#define TKV_KC(Dv, NBv)                                                                              \
-  do {                                                                                               \
-    if (f32) launch_key_blocks<Dv, NBv, true>(src, B, HKV, nblk, pos, start, S_cap, pk, sc, zr, st); \
-    else launch_key_blocks<Dv, NBv, false>(src, B, HKV, nblk, pos, start, S_cap, pk, sc, zr, st);    \
-  } while (0)
-  if (D == 128) {
-    if (nbits == 4) TKV_KC(128, 4); else TKV_KC(128, 2);
-  } else if (D == 64) {
-    if (nbits == 4) TKV_KC(64, 4); else TKV_KC(64, 2);
-  } else {
-    return TKV_EUNSUPPORTED;
-  }
-#undef TKV_KC
-  return TKV_OK;
+template <int D, int NB>
+static void launch_key_blocks(const void* x, bool f32, int B, int HKV, int nblk, const int32_t* pos,
+                              int S_cap, uint8_t* pk, uint16_t* sc, uint16_t* zr, hipStream_t st) {
+  const TokenSource src{x, (int64_t)HKV * nblk * 32 * D, (int64_t)nblk * 32 * D, D};
+  const bool wide = !((uintptr_t)x & (f32 ? 7 : 3));  // a lane's two channels in one load
+  const dim3 grid(key_workgroups<D>(HKV, nblk), (unsigned)(B < 65535 ? B : 65535));
+  if (f32)
+    quantize_keys_channel_kernel<D, NB, true><<<grid, 256, 0, st>>>(src, wide, B, HKV, nblk, pos, S_cap, pk, sc, zr);
+  else
+    quantize_keys_channel_kernel<D, NB, false><<<grid, 256, 0, st>>>(src, wide, B, HKV, nblk, pos, S_cap, pk, sc, zr);
+}
+
+template <int D, int NB>
+static void launch_channel_extend(const TokenSource& ks, const TokenSource& vs, int B, int HKV, int N,
+                                  int start, int S_cap, uint8_t* pk, uint16_t* sc, uint16_t* zr,
+                                  uint16_t* kr, uint16_t* vr, int32_t* ql, int32_t* rl, hipStream_t st) {
+  const int nblk = N / 32;
+  const unsigned wgs = key_workgroups<D>(HKV, nblk);
+  channel_extend_kernel<D, NB><<<dim3(wgs + HKV, (unsigned)B), 256, 0, st>>>(
+      ks, vs, (int)wgs, HKV, nblk, start, S_cap, pk, sc, zr, N % 32, kr, vr, ql, rl);
 }
 
 template <int D, int NB, int GS>
@@ -989,11 +1008,17 @@ extern "C" int tkv_quantize_keys_channel(const void* x, int32_t x_is_fp32, int32
   if ((uintptr_t)x & (x_is_fp32 ? 3 : 1)) return TKV_EINVAL;
   if ((int64_t)HKV * (N / T) > INT32_MAX) return TKV_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const TokenSource src{x, (int64_t)HKV * N * D, (int64_t)N * D, D};
   (void)hipGetLastError();
-  const int rc = launch_keys_channel(src, x_is_fp32 != 0, B, HKV, N / T, D, nbits, positions, 0,
-                                     S_cap, packed, scale, zero, st);
-  if (rc) return rc;
+#define TKV_KC(Dv, NBv) \
+  launch_key_blocks<Dv, NBv>(x, x_is_fp32 != 0, B, HKV, N / T, positions, S_cap, packed, scale, zero, st)
+  if (D == 128) {
+    if (nbits == 4) TKV_KC(128, 4); else TKV_KC(128, 2);
+  } else if (D == 64) {
+    if (nbits == 4) TKV_KC(64, 4); else TKV_KC(64, 2);
+  } else {
+    return TKV_EUNSUPPORTED;
+  }
+#undef TKV_KC
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? TKV_OK : (int)e;
 }
@@ -1040,10 +1065,17 @@ extern "C" int tkv_channel_extend(const void* k, const int64_t* k_strides, const
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   (void)hipGetLastError();
+#define TKV_CE(Dv, NBv)                                                                       \
+  launch_channel_extend<Dv, NBv>(ks, vs, B, HKV, N, start, S_cap, k_packed, k_scale, k_zero,  \
+                                 static_cast<uint16_t*>(k_res), static_cast<uint16_t*>(v_res), \
+                                 q_lens, res_lens, st)
+  if (D == 128) {
+    if (k_nbits == 4) TKV_CE(128, 4); else TKV_CE(128, 2);
+  } else {
+    if (k_nbits == 4) TKV_CE(64, 4); else TKV_CE(64, 2);
+  }
+#undef TKV_CE
   if (whole) {
-    const int rc = launch_keys_channel(ks, false, B, HKV, whole / T, D, k_nbits, nullptr, start, S_cap,
-                                       k_packed, k_scale, k_zero, st);
-    if (rc) return rc;
     bool done = false;
 #define TKV_VT(Dv, NBv, GSv) \
   done = launch_tokens<Dv, NBv, GSv>(vs, false, B, HKV, whole, nullptr, start, S_cap, v_packed, v_scale, v_zero, st)
@@ -1051,11 +1083,6 @@ extern "C" int tkv_channel_extend(const void* k, const int64_t* k_strides, const
 #undef TKV_VT
     if (!done) return TKV_EINVAL;
   }
-  const TokenSource kt{static_cast<const uint16_t*>(k) + whole * ks.st, ks.sb, ks.sh, ks.st};
-  const TokenSource vt{static_cast<const uint16_t*>(v) + whole * vs.st, vs.sb, vs.sh, vs.st};
-  channel_tail_kernel<<<dim3((unsigned)HKV, (unsigned)B), 256, 0, st>>>(
-      kt, vt, N - whole, D, static_cast<uint16_t*>(k_res), static_cast<uint16_t*>(v_res), q_lens,
-      res_lens, start + whole);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? TKV_OK : (int)e;
 }
