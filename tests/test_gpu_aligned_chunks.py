@@ -64,3 +64,25 @@ def test_short_rows_of_unaligned_blocks(nbits, HQ, S, append):
         assert torch.equal(got.scale.view(torch.int16), want.scale.view(torch.int16))
     ref = oracle_attention_on_quant(q, want_k, want_v, seq_lens=lens.cpu().numpy())
     assert_close_to_reference(out, ref, f"nbits={nbits} append={append}")
+
+
+@pytest.mark.parametrize("nbits,gs,HQ,S", [(4, 32, 8, 4127), (2, 32, 8, 8263), (4, 16, 32, 4099),
+                                           (2, 128, 8, 8250), (4, 32, 12, 8251)])
+def test_rows_before_the_block_do_not_show_what_lds_held(nbits, gs, HQ, S):
+    """The rows masked before a block's start are not loaded: a launch over a
+    cache of NaN scales and zero points leaves NaNs in every CU's LDS, and the
+    next launch must not see them."""
+    from tritonkv_amd.kernels import fused_decode_attention
+
+    B, HKV = 160, 2  # more workgroups than compute units
+    q, _, _, kq, vq = make_case(2, HQ, HKV, 128, S, nbits, gs, seed=S, outlier_frac=0.0)
+    wide = [t._map(lambda x: x[:1].expand(B, *x.shape[1:]).contiguous()) for t in (kq, vq)]
+    nan = [t._map(lambda x: x if x.dtype == torch.uint8 else torch.full_like(x, float("nan"))) for t in wide]
+    qs = q[:1].expand(B, -1, -1).contiguous()
+    want = fused_decode_attention(q[:1].contiguous(), *(t._map(lambda x: x[:1].contiguous())
+                                                        for t in (kq, vq)), num_splits=1)
+    assert not bool(want.isnan().any())
+    assert bool(fused_decode_attention(qs, *nan, num_splits=1).isnan().all())
+    got = fused_decode_attention(qs, *wide, num_splits=1)
+    assert not bool(got.isnan().any())
+    assert float((got - want).abs().max()) <= 2e-3

@@ -941,6 +941,18 @@ quant_split_lds_kernel(SplitParams prm) {
         *reinterpret_cast<uint16_t*>(sw + SG::M_OFF + (lane / NG) * SG::MB +
                                      2 * (t_new * SG::MROW + lane % NG)) = pmeta[lane];
     }
+    if constexpr (kAlign && SK == 0) {  // the wave's first chunk is in stage 0
+      // Rows before the split's start: the masked scores below give them p = 0,
+      // but loads out of the buffer range need not have written their scales
+      // and zero points, and what LDS held before can be a NaN.
+      if (cb < lo) {
+        uint8_t* sw = ring + SK * SG::BYTES + SG::M_OFF;
+        for (int i = lane; i < (lo - cb) * MR; i += 64)
+#pragma unroll
+          for (int tsr = 0; tsr < 4; ++tsr) *reinterpret_cast<uint16_t*>(sw + tsr * SG::MB + 2 * i) = 0;
+        wave_lds_fence();
+      }
+    }
     const uint8_t* st = ring + SK * SG::BYTES;
     const uint8_t* mks = st + SG::M_OFF;
     const uint8_t* mkz = mks + SG::MB;
@@ -1027,7 +1039,7 @@ quant_split_lds_kernel(SplitParams prm) {
         }
         }  // NG > 1
       }
-      if constexpr (kAlign && SK == 0)  // the wave's first chunk is in stage 0
+      if constexpr (kAlign && SK == 0)
         if (cb < lo) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
@@ -1209,7 +1221,7 @@ quant_split_lds_kernel(SplitParams prm) {
         }
       }
       }  // per-token key groups
-      if constexpr (kAlign && SK == 0)  // the wave's first chunk is in stage 0
+      if constexpr (kAlign && SK == 0)
         if (cb < lo) {
   #pragma unroll
           for (int a = 0; a < 2; ++a)
