@@ -124,8 +124,9 @@ def llama_inputs(seed, B=32, HQ=32, HKV=8, S=32768, D=128):
 
 
 # The split kernel's paired-tile form runs for GQA groups of at most 8 heads
-# and splits of at least this many tokens (kPairedTilesMinSplit in
-# tritonkv_amd/csrc/quant_split.h).
+# and splits of at least this many tokens; grids of a workgroup per compute unit
+# or more take it earlier (paired_tiles_min_split in
+# tritonkv_amd/csrc/quant_split.h), which no shape named here reaches.
 PAIRED_TILES_MIN_SPLIT = 8192
 
 

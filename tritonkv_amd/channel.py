@@ -186,8 +186,9 @@ def channel_decode_attention(
 
     group = HQ // HKV
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
-    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group,
-                                            ragged=q_lens is not None and not equal_lengths)
+    ragged = q_lens is not None and not equal_lengths
+    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged,
+                                            fine=False)
     q_in = q
     if q.dtype not in (torch.float16, torch.float32):
         q = q.float()
@@ -207,7 +208,8 @@ def channel_decode_attention(
         v_nbits=vq.nbits, group_size=vq.group_size, sm_scale=float(sm_scale),
         split_size=split_size, num_splits=num_splits, counters=None,
         waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, k_nbits=ck.nbits,
-                           v_nbits=vq.nbits, group_size=vq.group_size), key_block=BLOCK)
+                           v_nbits=vq.nbits, group_size=vq.group_size, ragged=ragged),
+        key_block=BLOCK)
     rc = _lib.launch(q.device, "tkv_channel_decode_attention", args, kr.data_ptr(), vr.data_ptr(),
                      _lib.ptr(rlens), R)
     _lib.check(rc, "channel_decode_attention")

@@ -1544,12 +1544,22 @@ void launch_quant_pt(const SplitParams& p, dim3 grid, int waves, hipStream_t st)
   launch_quant_pto<D, KNB, VNB, GS, PT, HS, false>(p, grid, waves, st);
 }
 
-// Paired tiles when the GQA group has at most 8 query heads and every
-// workgroup streams a long history.  They cost about 1 us more per workgroup
-// (twice the q operands to build, three more cross-lane moves per chunk), so
-// they pay only over many chunks per wave: measured 4-6% faster at 32768 tokens
-// per workgroup (2-bit, K4/V2), equal at 4096, 5-10% slower at 512-1024.
-constexpr int kPairedTilesMinSplit = 8192;
+// Split sizes from which paired tiles run, for GQA groups of at most 8 query
+// heads.  They issue a third less per chunk, but build twice the q operands per
+// wave (about 1 us), and their registers let two 4-wave workgroups share a CU
+// instead of three.  Grids of about a workgroup per CU or more (B = 32 or 64,
+// HKV = 8, 4-bit groups of 32, one split):
+//   8 waves  S = 512 8.5 -> 9.2 us, 2048 18.6 -> 18.0, 4096 30.6 -> 30.1
+//   4 waves  S = 1024 18.4 -> 18.0, 4096 55.5 -> 55.2 (2-bit 43.2 -> 39.8)
+// In a dispatch order (rows of different lengths) short rows pay the longer
+// prologue: 4 waves, pieces of 2048 42.2 -> 44.4 us, of 4096 72.9 -> 71.2.
+// Smaller grids keep the threshold of 8192 tokens: equal at 4096, 5-10%
+// slower at 512-1024, and a dims split is faster there.
+inline int paired_tiles_min_split(const SplitParams& p, dim3 grid, int waves) {
+  const unsigned long long wgs = 1ull * grid.x * grid.y * grid.z;
+  if (4 * wgs < 3ull * device_cus()) return 8192;
+  return waves <= 4 && p.order ? 4096 : 2048;
+}
 
 // ===========================================================================
 // Read-ceiling probe: what the split kernel's access pattern streams with no
@@ -1644,7 +1654,7 @@ void launch_quant_hs(const SplitParams& p, dim3 grid, int waves, hipStream_t st)
       return;
     }
   }
-  if (p.G <= 8 && p.split_size >= kPairedTilesMinSplit)
+  if (p.G <= 8 && p.split_size >= paired_tiles_min_split(p, grid, waves))
     launch_quant_pt<D, KNB, VNB, GS, true, HS>(p, grid, waves, st);
   else launch_quant_pt<D, KNB, VNB, GS, false, HS>(p, grid, waves, st);
 }

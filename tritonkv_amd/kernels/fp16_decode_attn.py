@@ -84,9 +84,9 @@ def fp16_decode_attention(
 
     group = HQ // HKV
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
+    ragged = seq_lens is not None and not equal_lengths
     _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group,
-                                            TOKENS_PER_WORKGROUP_FP16,
-                                            ragged=seq_lens is not None and not equal_lengths)
+                                            TOKENS_PER_WORKGROUP_FP16, ragged=ragged, fine=False)
 
     q_in = q
     if q.dtype not in (torch.float16, torch.float32):
@@ -105,7 +105,7 @@ def fp16_decode_attention(
         acc=_lib.ptr(acc), maxs=_lib.ptr(maxs), sums=_lib.ptr(sums), out=out.data_ptr(),
         B=B, HQ=HQ, HKV=HKV, S=S, D=D, k_nbits=16, v_nbits=16, group_size=D,
         sm_scale=float(sm_scale), split_size=split_size, num_splits=num_splits,
-        counters=None, waves=choose_waves(B, HKV, group, split_size, num_splits))
+        counters=None, waves=choose_waves(B, HKV, group, split_size, num_splits, ragged=ragged))
     rc = _lib.launch(q.device, "tkv_fp16_decode_attention", args)
     _lib.check(rc, "fp16_decode_attention")
     # k / v are read in place; a converted copy (not fp16, not contiguous) is not kept

@@ -118,7 +118,7 @@ MAX_SPLITS = 65535  # grid y-dimension limit
 
 def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
                        tokens_per_workgroup: int = TOKENS_PER_WORKGROUP, *,
-                       ragged: bool = False) -> int:
+                       ragged: bool = False, fine: bool = True) -> int:
     """Split count used when the caller passes ``num_splits=None``.
 
     Chosen from sweeps on MI355X (split count x workgroup size, DRAM-resident
@@ -154,6 +154,18 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
     unsplit.  Equal lengths pay for the second split (Llama-3-8B shape:
     206.6 vs 200.7 us).
 
+    ``fine``: the caller runs short ragged pieces in 4-wave workgroups
+    (``choose_waves``), of which a CU holds two or three, so that a finer cut
+    costs little and evens out rows of different lengths (K4/V2, G = 8, in us):
+
+    * half a unit to one unit per CU: 4 workgroups per CU in pieces of at least
+      1024 tokens (24 rows of up to 32768: 111.8 at 1 split -> 84-90 at 4-8;
+      20 rows of up to 4096: 22.3 -> 20.0; 16 rows of up to 8192: 26.7 -> 24.5;
+      16 rows of up to 2048: 13.4 either way at best, so not below 4096);
+    * one to two units per CU and 65536 tokens or more: pieces of 8192-16384
+      tokens (32 rows of up to 65536: 174 at 2 splits -> 172 at 6, 2-bit 143 ->
+      133, 4-bit 205 -> 201).
+
     Returned in units of ``block_n`` blocks so the reference's tightening
     applies unchanged.
     """
@@ -164,7 +176,10 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
     if units >= cu:
         if not ragged or S < 16384:
             return 1
-        return min(max(2, S // 32768), _cdiv(S, block_n))
+        piece = 32768 if units >= 2 * cu or S < 65536 or not fine else 10922
+        return min(max(2, S // piece), _cdiv(S, block_n))
+    if ragged and fine and 2 * units >= cu and S >= 4096:
+        return max(1, min(4 * cu // units, S // 1024, _cdiv(S, block_n)))
     workgroups = min(cu, max(32, units * S // tokens_per_workgroup))
     want = max(1, workgroups // units)
     max_splits = max(1, S // max(tokens_per_workgroup // 4, block_n))
@@ -193,12 +208,31 @@ def twelve_wave_format(D: int, G: int, k_nbits: int, v_nbits: int, group_size: i
 
 def choose_waves(B: int, HKV: int, G: int, split_size: int, num_splits: int = 0, *,
                  D: int = 128, k_nbits: int = 16, v_nbits: int = 16, group_size: int = 0,
-                 paged: bool = False) -> int:
-    """Waves per workgroup: 12 for the formats of ``twelve_wave_format`` when a
+                 paged: bool = False, ragged: bool = False) -> int:
+    """Waves per workgroup.
+
+    4 when the grid holds at least one and a half workgroups per compute unit
+    and none streams more than 32768 tokens: a CU then holds two or three of
+    them at once, and one streams while another builds its q operands or merges
+    (an 8-wave workgroup fills a CU's LDS or registers alone).  HKV = 8, G = 4,
+    8 or 12 waves -> 4, us: B = 64 4-bit ctx 1024 21.8 -> 18.0, 4096 58.9 ->
+    55.2, 16384 205.3 -> 201.5; 2-bit ctx 4096 45.9 -> 39.8, 16384 142 -> 134;
+    B = 128 ctx 1024 42.7 -> 33.3; at one workgroup per CU 2-bit ctx 4096
+    22.7 -> 24.6.  With rows of different lengths (``ragged``) fewer, larger
+    workgroups balance better until there are many pieces or they are short:
+    4 waves from four workgroups per CU (64 rows of up to 131072, 4 splits
+    647 -> 630) or for pieces of at most 4096 tokens (64 rows of up to 1024
+    21.2 -> 14.3, 4096 41.4 -> 40.6, but 8192 63.2 -> 69.3).
+
+    Otherwise 12 for the formats of ``twelve_wave_format`` when a
     workgroup streams at least ``TWELVE_WAVES_MIN_SPLIT`` tokens; else 8 when
     it streams the whole history or at least 512 tokens (two 32-token chunks
     per wave, so each wave overlaps a load with compute); else 4.  The default
     format (16-bit) is the fp16 control's."""
+    wgs, cu = B * HKV * _cdiv(G, 16) * num_splits, compute_units() or 256
+    if 2 * wgs >= 3 * cu and split_size <= 32768 and \
+            (not ragged or wgs >= 4 * cu or split_size <= 4096):
+        return 4
     if split_size >= TWELVE_WAVES_MIN_SPLIT and \
             twelve_wave_format(D, G, k_nbits, v_nbits, group_size, paged):
         return 12
@@ -206,7 +240,8 @@ def choose_waves(B: int, HKV: int, G: int, split_size: int, num_splits: int = 0,
 
 
 def plan_splits(S: int, block_n: int, num_splits: int | None, B: int, HKV: int, G: int,
-                tokens_per_workgroup: int = TOKENS_PER_WORKGROUP, *, ragged: bool = False):
+                tokens_per_workgroup: int = TOKENS_PER_WORKGROUP, *, ragged: bool = False,
+                fine: bool = True):
     """Reference split arithmetic (:486-499) -> (block_n, num_splits, split_size).
 
     One addition: the count is capped at 65535 before tightening (splits are
@@ -215,7 +250,7 @@ def plan_splits(S: int, block_n: int, num_splits: int | None, B: int, HKV: int, 
     n_blocks = _cdiv(S, block_n)
     if num_splits is None:
         num_splits = default_num_splits(B, HKV, G, S, block_n, tokens_per_workgroup,
-                                        ragged=ragged)
+                                        ragged=ragged, fine=fine)
     num_splits = max(1, min(num_splits, n_blocks, MAX_SPLITS))
     blocks_per_split = _cdiv(n_blocks, num_splits)
     num_splits = _cdiv(n_blocks, blocks_per_split)  # tighten: no empty splits
@@ -255,14 +290,21 @@ def _workspace_for(ws: dict | None, B: int, HQ: int, num_splits: int, D: int, de
 # The order kernel ranks each piece against every row (O(B) per piece, so
 # O(B^2 * num_splits) in all); the automatic order stops at this many rows.
 ORDER_MAX_ROWS = 2048
+# Shortest pieces the automatic order is taken for: its launch (3-5 us) is more
+# than it saves on shorter ones (us without -> with it: 64 rows of up to 2048
+# 24.0 -> 26.2, 128 rows of up to 4096 68.5 -> 68.7, 16 rows of up to 8192 in
+# pieces of 1024 25.3 -> 28.4; 64 rows of up to 8192 71.1 -> 63.2).
+ORDER_MIN_PIECE = 4096
 
 
 def _order_for(ws: dict | None, B: int, HKV: int, num_splits: int, device, seq_lens,
-               dispatch_order: bool | None, G: int = 1, D: int = 128):
+               dispatch_order: bool | None, G: int = 1, D: int = 128,
+               split_size: int | None = None):
     """The ``work_order`` buffer of a split call, or None.
 
     ``dispatch_order=None`` takes it when ``seq_lens`` is given, the batch
-    has at most ``ORDER_MAX_ROWS`` rows and the grid holds more workgroups
+    has at most ``ORDER_MAX_ROWS`` rows, the pieces (``split_size``) hold at
+    least ``ORDER_MIN_PIECE`` tokens and the grid holds more workgroups
     than the GPU has compute units: the call then runs the split workgroups
     longest piece first (``ragged_order_kernel``), which evens out the end of
     the launch when rows differ in length (B=64, HKV=8, lengths U[1k, 128k],
@@ -278,7 +320,8 @@ def _order_for(ws: dict | None, B: int, HKV: int, num_splits: int, device, seq_l
     if dispatch_order is None:
         workgroups = B * HKV * _cdiv(G, 16) * num_splits
         if seq_lens is None or workgroups <= (compute_units(device) or 256) \
-                or B > ORDER_MAX_ROWS or D != 128:
+                or B > ORDER_MAX_ROWS or D != 128 \
+                or (split_size is not None and split_size < ORDER_MIN_PIECE):
             return None
     ws = ws if ws is not None else {}
     n = 2 * B * HKV * num_splits  # (s * B * HKV + unit, row length) pairs
@@ -518,7 +561,7 @@ def fused_decode_attention(
     acc, maxs, sums, counters = _workspace_for(_workspace, B, HQ, num_splits, D, q.device, HKV)
     lens = _seq_lens_arg(seq_lens, B, S, q.device)
     order = _order_for(_workspace, B, HKV, num_splits, q.device, seq_lens if ragged else None,
-                       dispatch_order, group, D)
+                       dispatch_order, group, D, split_size)
 
     args = _lib.DecodeArgs(
         q=q.data_ptr(), q_is_fp32=int(q.dtype == torch.float32),
@@ -530,7 +573,7 @@ def fused_decode_attention(
         sm_scale=float(sm_scale), split_size=split_size, num_splits=num_splits,
         counters=_lib.ptr(counters) if fused_combine else None,
         waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, k_nbits=kq.nbits,
-                           v_nbits=vq.nbits, group_size=kq.group_size),
+                           v_nbits=vq.nbits, group_size=kq.group_size, ragged=ragged),
         k_new=_lib.ptr(kn), v_new=_lib.ptr(vn), new_is_fp32=new_f32,
         work_order=_lib.ptr(order))
     rc = _lib.launch(q.device, "tkv_fused_decode_attention", args)

@@ -188,7 +188,7 @@ def paged_decode_attention(
     acc, maxs, sums, counters = _workspace_for(_workspace, B, HQ, num_splits, D, q.device, HKV)
     lens = seq_lens.contiguous() if seq_lens is not None else None
     order = _order_for(_workspace, B, HKV, num_splits, q.device, seq_lens if ragged else None,
-                       dispatch_order, group, D)
+                       dispatch_order, group, D, split_size)
     args = _lib.DecodeArgs(
         q=q.data_ptr(), q_is_fp32=int(q.dtype == torch.float32),
         k=k_pool.packed.data_ptr(), k_scale=k_pool.scale.data_ptr(),
@@ -199,7 +199,7 @@ def paged_decode_attention(
         k_nbits=k_pool.nbits, v_nbits=v_pool.nbits, group_size=k_pool.group_size,
         sm_scale=float(sm_scale), split_size=split_size, num_splits=num_splits, counters=None,
         waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, k_nbits=k_pool.nbits,
-                           v_nbits=v_pool.nbits, group_size=k_pool.group_size, paged=True),
+                           v_nbits=v_pool.nbits, group_size=k_pool.group_size, paged=True, ragged=ragged),
         block_table=table.data_ptr(), block_table_stride=table.shape[1], page_size=page_size,
         num_pages=num_pages, k_new=_lib.ptr(kn), v_new=_lib.ptr(vn), new_is_fp32=new_f32,
         work_order=_lib.ptr(order))
