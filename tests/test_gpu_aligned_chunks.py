@@ -86,3 +86,19 @@ def test_rows_before_the_block_do_not_show_what_lds_held(nbits, gs, HQ, S):
     got = fused_decode_attention(qs, *wide, num_splits=1)
     assert not bool(got.isnan().any())
     assert float((got - want).abs().max()) <= 2e-3
+
+
+@pytest.mark.parametrize("fused_combine,ns", [(False, 1), (True, 2)])
+def test_empty_rows_and_splits_of_unaligned_blocks(fused_combine, ns):
+    """A row or split with no tokens runs no chunk, as where S is a multiple of 32."""
+    from tritonkv_amd.kernels import fused_decode_attention
+
+    B, S = 4, 8251
+    q, _, _, kq, vq = make_case(B, 8, 2, 128, S, 4, 32, seed=5, outlier_frac=0.0)
+    lens = torch.tensor([0, 4000, 0, S], dtype=torch.int32, device=DEV)
+    even = [t._map(lambda x: torch.cat([x, x[:, :, :-S % 32]], 2).contiguous()) for t in (kq, vq)]
+    got, want = (fused_decode_attention(q, *c, seq_lens=lens, num_splits=ns, fused_combine=fused_combine)
+                 for c in ((kq, vq), even))
+    assert torch.equal(got[::2].isnan(), want[::2].isnan())
+    assert torch.equal(got[::2].nan_to_num(), want[::2].nan_to_num())
+    assert float((got[1::2] - want[1::2]).abs().max()) <= 2e-3

@@ -33,8 +33,9 @@ struct StageGeom {
   // fp16 slots per token row of a staged metadata tensor: the global row of NG
   // values, except NG == 1: a chunk whose rows all lie before the split's last
   // token is copied as whole dwords (fp16 pairs of tokens 2i, 2i + 1, MROW_PAIRS
-  // = 1), the chunk holding the last token one fp16 per dword (MROW = 2: a dword
-  // copy could straddle the end of the buffer range there).
+  // = 1), the chunk holding the last token and a first one that reaches before the
+  // split one fp16 per dword (MROW = 2: a dword copy could straddle an end of
+  // the buffer range there).
   static constexpr int MROW = NG >= 2 ? NG : 2;
   static constexpr int MROW_PAIRS = NG >= 2 ? NG : 1;
   static constexpr int KB = kChunk * KL::DP;    // K code bytes per chunk
@@ -610,14 +611,15 @@ quant_split_lds_kernel(SplitParams prm) {
     }
 
   // Chunk k of this wave starts at token lo - head + 32 * (w + NW * k); the
-  // split's first chunk masks the `head` rows before lo (SplitParams::row_align).
+  // split's first chunk masks the `head` rows before lo (SplitParams::row_align;
+  // `early` below).
   constexpr bool kAlign = !PAGED && !KCH && VS == 1;
   const int first = lo - (kAlign ? (int)(((uint32_t)unit * (uint32_t)prm.S + (uint32_t)lo) &
                                          (uint32_t)prm.row_align)
                                  : 0);
   const int cb0 = first + kChunk * w;
   const int cstride = kChunk * NW;
-  static_assert(NSTAGE >= 2 && (!PAGED || NSTAGE == 2), "ring depth");
+  static_assert(NSTAGE >= 2 && (!(PAGED || kAlign) || NSTAGE == 2), "ring depth");
   // Paged: page_next is the pool page of the chunk whose DMA is issued next;
   // tab_pending the (in-flight) table entry of the chunk after that.
   int page_next = 0;
@@ -631,13 +633,15 @@ quant_split_lds_kernel(SplitParams prm) {
                                       cb0 + kChunk < hi);
     tab_pending = tab_entry(cb0 + 2 * cstride);
   } else {
-    // the first NSTAGE - 1 chunks into stages 0 .. NSTAGE - 2
+    // the first NSTAGE - 1 chunks into stages 0 .. NSTAGE - 2; a chunk that
+    // reaches before the split into the last stage (see stream)
     static_for<NSTAGE - 1>([&](auto s) __attribute__((always_inline)) {
       constexpr int SS = decltype(s)::value;
       const int c = cb0 + SS * cstride;
+      const bool early = kAlign && c < lo;
       const ChunkSrc src = chunk_src(c, 0);
-      issue_chunk<D, KNB, VNB, GS, KCH>(ring + SS * SG::BYTES, src.k, src.v, src.m, src.row, c < hi, lane,
-                                        c + kChunk < hi);
+      issue_chunk<D, KNB, VNB, GS, KCH>(ring + (early ? NSTAGE - 1 : SS) * SG::BYTES, src.k, src.v, src.m,
+                                        src.row, c < hi, lane, c + kChunk < hi && !early);
     });
   }
 
@@ -868,15 +872,24 @@ quant_split_lds_kernel(SplitParams prm) {
   asm volatile("" : "+v"(zero_v));
   const float lscale = prm.qk_scale * __builtin_ldexpf(1.0f, 24 - eh);  // per lane (its head)
 
-  // A row before the split's start takes a score no key reaches.  It is
-  // finite, so a chunk whose other scores are all -inf keeps a finite maximum.
-  constexpr float x_head = -1e30f;
-
-  // In the tail chunk, rows past the sequence hold whatever the cache holds
-  // there (possibly NaN/Inf bit patterns in scale/zero): their V scale and
-  // zero-point pairs are cleared, since p = 0 alone would not cancel them.
-  auto tail_pair_mask = [&](int tok0, int tok1) -> uint32_t {
-    return (tok0 <= last ? 0x0000FFFFu : 0u) | (tok1 <= last ? 0xFFFF0000u : 0u);
+  // The TAIL step masks the rows past the sequence, and its `early` form, for a
+  // split's first chunk that reaches before the split (kAlign), those there too.
+  // A row before the split takes a score no key reaches; it is finite, so a
+  // chunk whose other scores are all -inf keeps a finite maximum.
+  auto mask_row = [&](float& x, int tok, auto early) {
+    if (tok > last) x = -INFINITY;
+    if (decltype(early)::value && tok < lo) x = -1e30f;
+  };
+  auto masked = [&](int tok, auto early) -> bool {
+    if constexpr (decltype(early)::value) return (uint32_t)(tok - lo) > (uint32_t)(last - lo);
+    else return tok > last;
+  };
+  // Masked rows hold whatever the cache holds there (possibly NaN/Inf bit
+  // patterns in scale/zero), or whatever LDS held (a load out of a resource's
+  // range need not write): their V scale and zero-point pairs are cleared,
+  // since p = 0 alone would not cancel them.
+  auto tail_pair_mask = [&](int tok0, int tok1, auto early) -> uint32_t {
+    return (masked(tok0, early) ? 0u : 0x0000FFFFu) | (masked(tok1, early) ? 0u : 0xFFFF0000u);
   };
   auto half_at = [&](const uint8_t* base, int idx) -> uint32_t {  // fp16 bits of element idx
     return *reinterpret_cast<const uint16_t*>(base + 2 * idx);
@@ -888,8 +901,9 @@ quant_split_lds_kernel(SplitParams prm) {
 
   // Chunk k of the wave uses stage k % NSTAGE; the loop below is unrolled by
   // NSTAGE so every stage offset is a compile-time constant.
-  auto step = [&](int cb, auto tail, auto stage, auto pmode, auto part) __attribute__((always_inline)) {
+  auto step = [&](int cb, auto tail, auto stage, auto pmode, auto part, auto early) __attribute__((always_inline)) {
     constexpr bool TAIL = decltype(tail)::value;
+    constexpr bool EARLY = decltype(early)::value;  // see mask_row; always with TAIL
     constexpr int SK = decltype(stage)::value;
     constexpr int PART = decltype(part)::value;  // dims part (VS > 1)
     // hi/lo probabilities in the PV products (see kHiLoMaxLen)
@@ -913,7 +927,7 @@ quant_split_lds_kernel(SplitParams prm) {
       const int cn = cb + (NSTAGE - 1) * cstride;
       wait_lgkmcnt0();  // the previous chunk's LDS reads of that stage are done
       asm volatile("" ::: "memory");
-      const bool valid = !TAIL && cn < hi;
+      const bool valid = (EARLY || !TAIL) && cn < hi;
       const ChunkSrc src = chunk_src(cn, page_next);
       issue_chunk<D, KNB, VNB, GS, KCH>(ring + ((SK + NSTAGE - 1) % NSTAGE) * SG::BYTES, src.k, src.v,
                                    src.m, src.row, valid, lane, cn + kChunk < hi);
@@ -940,18 +954,6 @@ quant_split_lds_kernel(SplitParams prm) {
       if (lane < 4 * NG)
         *reinterpret_cast<uint16_t*>(sw + SG::M_OFF + (lane / NG) * SG::MB +
                                      2 * (t_new * SG::MROW + lane % NG)) = pmeta[lane];
-    }
-    if constexpr (kAlign && SK == 0) {  // the wave's first chunk is in stage 0
-      // Rows before the split's start: the masked scores below give them p = 0,
-      // but loads out of the buffer range need not have written their scales
-      // and zero points, and what LDS held before can be a NaN.
-      if (cb < lo) {
-        uint8_t* sw = ring + SK * SG::BYTES + SG::M_OFF;
-        for (int i = lane; i < (lo - cb) * MR; i += 64)
-#pragma unroll
-          for (int tsr = 0; tsr < 4; ++tsr) *reinterpret_cast<uint16_t*>(sw + tsr * SG::MB + 2 * i) = 0;
-        wave_lds_fence();
-      }
     }
     const uint8_t* st = ring + SK * SG::BYTES;
     const uint8_t* mks = st + SG::M_OFF;
@@ -1022,7 +1024,7 @@ quant_split_lds_kernel(SplitParams prm) {
           // rows past the sequence (whatever the cache holds there) are cleared
           // so they cannot reach the other tile's columns.
           if constexpr (TAIL)
-            if (cb + 16 * (j >> 1) + r > last) za = u4{0u, 0u, 0u, 0u};
+            if (masked(cb + 16 * (j >> 1) + r, early)) za = u4{0u, 0u, 0u, 0u};
         }
         const f4 yz = mfma_k32(za, qpt.qzb, f4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
@@ -1039,16 +1041,9 @@ quant_split_lds_kernel(SplitParams prm) {
         }
         }  // NG > 1
       }
-      if constexpr (kAlign && SK == 0)
-        if (cb < lo) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (cb + tile_pt + 4 * j + i < lo) x[i] = x_head;
-        }
       if constexpr (TAIL) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (cb + tile_pt + 4 * j + i > last) x[i] = -INFINITY;
+        for (int i = 0; i < 4; ++i) mask_row(x[i], cb + tile_pt + 4 * j + i, early);
       }
       // ---- online softmax ---------------------------------------------------
       float alpha;
@@ -1221,20 +1216,11 @@ quant_split_lds_kernel(SplitParams prm) {
         }
       }
       }  // per-token key groups
-      if constexpr (kAlign && SK == 0)
-        if (cb < lo) {
-  #pragma unroll
-          for (int a = 0; a < 2; ++a)
-  #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (cb + 16 * a + 4 * j + i < lo) x[4 * a + i] = x_head;
-        }
       if constexpr (TAIL) {
   #pragma unroll
         for (int a = 0; a < 2; ++a)
   #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (cb + 16 * a + 4 * j + i > last) x[4 * a + i] = -INFINITY;
+          for (int i = 0; i < 4; ++i) mask_row(x[4 * a + i], cb + 16 * a + 4 * j + i, early);
       }
 
       // ---- online softmax ---------------------------------------------------
@@ -1269,7 +1255,7 @@ quant_split_lds_kernel(SplitParams prm) {
           zp[q] = perm(*reinterpret_cast<const uint32_t*>(mvz + zoff + 2 * t1 * MR),
                        *reinterpret_cast<const uint32_t*>(mvz + zoff + 2 * t0 * MR), zsel);
         }
-        if constexpr (TAIL) zp[q] &= tail_pair_mask(cb + t0, cb + t1);
+        if constexpr (TAIL) zp[q] &= tail_pair_mask(cb + t0, cb + t1, early);
       }
       oz = mfma_k32(u4{zp[0], zp[1], zp[2], zp[3]}, pb, oz);
       if constexpr (HILO) oz = mfma_k32(u4{zp[0], zp[1], zp[2], zp[3]}, pbl, oz);
@@ -1291,7 +1277,7 @@ quant_split_lds_kernel(SplitParams prm) {
           const uint32_t d1 = *reinterpret_cast<const uint32_t*>(mvs + 2 * t1 * MR + soff[v]);
           sp[q] = perm(d1, d0, ssel[v]);
         }
-        if constexpr (TAIL) sp[q] &= tail_pair_mask(cb + t0, cb + t1);
+        if constexpr (TAIL) sp[q] &= tail_pair_mask(cb + t0, cb + t1, early);
       }
       pg[v] = u4{pk_mul(pb[0], sp[0]), pk_mul(pb[1], sp[1]), pk_mul(pb[2], sp[2]), pk_mul(pb[3], sp[3])};
       if constexpr (HILO) {
@@ -1361,19 +1347,29 @@ quant_split_lds_kernel(SplitParams prm) {
   // across the unrolled copies.
   auto stream = [&](auto pmode, auto part) __attribute__((always_inline)) {
     int cb = cb0;
+    // A first chunk that reaches before the split: a masked copy of the step, in
+    // the last stage, so that the loop starts at stage 0 and carries no mask (a
+    // mask under a branch inside it cost 0.3-1.5% where no chunk takes it).
+    if constexpr (kAlign) {
+      if (cb < lo) {
+        if (lo < hi)  // an empty row or split has no chunk
+          step(cb, std::true_type{}, std::integral_constant<int, NSTAGE - 1>{}, pmode, part, std::true_type{});
+        cb += cstride;
+      }
+    }
     for (; cb + (NSTAGE - 1) * cstride + kChunk < hi; cb += NSTAGE * cstride) {
       static_for<NSTAGE>([&](auto s) __attribute__((always_inline)) {
-        step(cb + decltype(s)::value * cstride, std::false_type{}, s, pmode, part);
+        step(cb + decltype(s)::value * cstride, std::false_type{}, s, pmode, part, std::false_type{});
       });
     }
     bool more = true;
     static_for<NSTAGE>([&](auto s) __attribute__((always_inline)) {
       if (more) {
         if (cb + kChunk < hi) {
-          step(cb, std::false_type{}, s, pmode, part);
+          step(cb, std::false_type{}, s, pmode, part, std::false_type{});
           cb += cstride;
         } else {
-          if (cb < hi) step(cb, std::true_type{}, s, pmode, part);
+          if (cb < hi) step(cb, std::true_type{}, s, pmode, part, std::false_type{});
           more = false;
         }
       }
