@@ -114,3 +114,19 @@ def test_channel_cache_checks_token_shapes_before_any_launch():
     c._rlens.fill_(5)
     c.reset()
     assert len(c) == 0 and not c._qlens.any() and not c._rlens.any()
+
+
+@pytest.mark.parametrize("held,n", [(0, 32), (0, 40), (5, 27), (5, 60)])
+def test_a_cpu_cache_refuses_what_would_flush_before_it_writes(held, n):
+    from tritonkv_amd.channel import ChannelKVCache
+
+    c = ChannelKVCache(2, 2, 128, 128, device="cpu")
+    x = torch.randn(2, 2, 64, 128).to(torch.float16)
+    c.extend(x[:, :, :held], x[:, :, :held])
+    before = c.k_res.clone(), c.v_res.clone()
+    with pytest.raises(RuntimeError, match="GPU"):
+        c.extend(x[:, :, :n], x[:, :, :n])
+    assert (c.quantized, c.window) == (0, held) and not c._qlens.any() and (c._rlens == held).all()
+    assert torch.equal(c.k_res, before[0]) and torch.equal(c.v_res, before[1])
+    c.extend(x[:, :, held:held + 3], x[:, :, held:held + 3])  # still usable
+    assert len(c) == held + 3 and torch.equal(c.k_res[:, :, :held + 3], x[:, :, :held + 3])

@@ -318,6 +318,8 @@ class ChannelKVCache:
         N = k.shape[2]
         if len(self) + N > self.capacity:
             raise ValueError(f"cache capacity {self.capacity} exceeded ({len(self)} + {N})")
+        if self.window + N >= BLOCK:  # quantizes: nothing is written where that cannot run
+            _require_gpu(k, "ChannelKVCache.extend")
         i = 0
         if (self.window and N) or not k.is_cuda:  # fill the open window first
             i = min(BLOCK - self.window, N)
