@@ -102,3 +102,31 @@ def test_empty_rows_and_splits_of_unaligned_blocks(fused_combine, ns):
     assert torch.equal(got[::2].isnan(), want[::2].isnan())
     assert torch.equal(got[::2].nan_to_num(), want[::2].nan_to_num())
     assert float((got[1::2] - want[1::2]).abs().max()) <= 2e-3
+
+
+@pytest.mark.parametrize("kb,vb,gs,HQ,S", [
+    (4, 4, 32, 8, 16411),   # paired tiles, two splits of 8256
+    (2, 2, 32, 8, 16417),   # 12 waves; S % 32 == 1, so unit 1 starts one row into its chunk
+    (4, 2, 32, 16, 16385),  # 8 head columns
+    (4, 4, 16, 40, 8225),   # two blocks of 16 query heads, one tile at a time, splits of 4160
+    (2, 4, 64, 2, 16390),   # one query head
+])
+def test_later_splits_and_ordered_launches_of_unaligned_blocks(kb, vb, gs, HQ, S):
+    """Second splits that start inside a chunk, rows that end in that chunk, at
+    its start and one row past it; the ordered kernels bit for bit the same."""
+    from tritonkv_amd.kernels import fused_decode_attention
+    from tritonkv_amd.kernels.fused_decode_attn import plan_splits
+    from tritonkv_amd.quantize import quantize_groupwise
+
+    HKV = 2
+    print(f"aligned splits K{kb}V{vb} gs{gs} HQ={HQ} S={S}", flush=True)
+    q, _, v, kq, _ = make_case(5, HQ, HKV, 128, S, kb, gs, seed=S, outlier_frac=0.0)
+    vq = quantize_groupwise(v, vb, gs)
+    lo = plan_splits(S, 64, 2, 5, HKV, HQ // HKV)[2]
+    lens = torch.tensor([S, lo, lo + 1, lo + 3, lo + 40], dtype=torch.int32, device=DEV)
+    outs = [fused_decode_attention(q, kq, vq, seq_lens=lens, num_splits=2, allow_mixed_bits=kb != vb,
+                                   dispatch_order=order, _workspace={}) for order in (False, True)]
+    torch.cuda.synchronize()
+    assert torch.equal(*outs)
+    assert_close_to_reference(outs[0], oracle_attention_on_quant(q, kq, vq, seq_lens=lens.cpu().numpy()),
+                              f"K{kb}V{vb} gs{gs} S={S}")

@@ -215,3 +215,27 @@ def test_equal_lengths_take_the_unragged_plan(monkeypatch, length):
         out_none = fda.fused_decode_attention(q, kq, vq)
         torch.cuda.synchronize()
         assert torch.equal(out_eq, out_none)
+
+
+@pytest.mark.parametrize("B,HQ,HKV,S,nbits,ns", [
+    (1, 12, 2, 5001, 4, 1),      # a dims-split grid whose blocks start inside a cache line
+    (1, 12, 2, 9001, 2, 2),
+    (4, 12, 2, 8101, 4, 1),
+])
+def test_the_order_and_the_merge_do_not_choose_the_kernel_form(B, HQ, HKV, S, nbits, ns):
+    """Tile form and chunk starts follow from the grid, the split and the
+    format, so that neither an order nor counters change the output's bits."""
+    from tritonkv_amd.kernels import fused_decode_attention
+
+    print(f"forms B={B} HQ={HQ} HKV={HKV} S={S} nbits={nbits} ns={ns}", flush=True)
+    q, _, _, kq, vq = make_case(min(B, 5), HQ, HKV, 128, S, nbits, 32, seed=S)
+    rows = torch.arange(B, device=DEV) % q.shape[0]
+    q, kq, vq = q[rows], kq._map(lambda t: t[rows]), vq._map(lambda t: t[rows])
+    lens = _lengths(B, S, 64, seed=S).to(DEV)
+    outs = [fused_decode_attention(q, kq, vq, num_splits=ns, seq_lens=lens, dispatch_order=order,
+                                   fused_combine=merge, _workspace={})
+            for merge in (False, True) for order in (False, True)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[3], outs[2])
+    if ns != 2:  # a combine launch adds its partials in another order than the merge
+        assert torch.equal(outs[2], outs[0])

@@ -539,29 +539,6 @@ static int64_t range_rows(const tkv_decode_args* a) {
   return a->page_size > 0 ? a->page_size : a->S;
 }
 
-// Whether chunks start at multiples of 32 rows of the tensor (SplitParams::
-// row_align).  Where S is no multiple of 32, a (b, kv head) block starts
-// inside a cache line, and chunks counted from its start load pieces of one
-// more line per tensor each (B = 32, HKV = 8, D = 128, groups of 32: 4-bit at
-// S = 32767 225.9 -> 204.2 us, against 200.3 at 32768; 2-bit at S = 24571
-// 111.9 -> 102.9, against 101.4 at 24576).  An aligned split has up to one
-// more chunk, and its first is masked below the split's start, so it pays for
-// splits that stream many chunks (B = 16, S = 8191, 8 waves, 4-bit: 32.2 ->
-// 31.0 us at 4096 tokens a split, 35.8 -> 34.9 at 2048, 42.8 -> 42.9 at 1024;
-// 2-bit 23.7 -> 23.2, and no change below).  The masked rows of the first
-// split lie before the block: their offsets wrap past the 32-bit range check,
-// which needs blocks below 2^31 bytes; pairs of one-group rows' metadata must
-// not straddle the block's start (even S), and the mask is a large negative
-// score (a positive scale).
-constexpr int kAlignMinSplit = 4096;
-
-static bool aligned_chunks(const tkv_decode_args* a) {
-  if (a->S % 32 == 0 || a->page_size > 0 || a->key_block || a->split_size < kAlignMinSplit) return false;
-  if (!(a->sm_scale > 0.0f) || a->group_size <= 0) return false;
-  if (a->group_size == a->D && a->S % 2) return false;
-  return (int64_t)a->S * a->D < (int64_t(1) << 31);  // codes and metadata are smaller
-}
-
 static SplitParams make_params(const tkv_decode_args* a) {
   SplitParams p;
   p.q = a->q;
@@ -597,7 +574,6 @@ static SplitParams make_params(const tkv_decode_args* a) {
   p.ns_total = a->num_splits_total ? a->num_splits_total : a->num_splits;
   p.order = nullptr;  // set by launch_fused_split once the order is written
   p.xcd_units = 0;   // set by the small-grid dims-split launch
-  p.row_align = aligned_chunks(a) ? 31 : 0;
   return p;
 }
 

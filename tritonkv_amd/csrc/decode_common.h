@@ -3,6 +3,8 @@
 // q operands of the quantized kernel.
 #pragma once
 
+#include <limits.h>
+
 #include <type_traits>
 #include <utility>
 
@@ -56,10 +58,6 @@ struct SplitParams {
   // other launch (a flag in the argument block, which the prologue loads
   // anyway: the grid's own size would be another load).
   int xcd_units;
-  // Chunk alignment (quantized path): with 31, a split's chunks start at
-  // multiples of 32 rows of the whole tensor, not of the split, so that chunk
-  // loads fall on whole cache lines whatever S is; 0: at the split's start.
-  int row_align;
 };
 
 // Longest piece first: the dispatch order ragged_order_kernel writes.  Piece

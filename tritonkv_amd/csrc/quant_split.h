@@ -33,9 +33,8 @@ struct StageGeom {
   // fp16 slots per token row of a staged metadata tensor: the global row of NG
   // values, except NG == 1: a chunk whose rows all lie before the split's last
   // token is copied as whole dwords (fp16 pairs of tokens 2i, 2i + 1, MROW_PAIRS
-  // = 1), the chunk holding the last token and a first one that reaches before the
-  // split one fp16 per dword (MROW = 2: a dword copy could straddle an end of
-  // the buffer range there).
+  // = 1), the chunk holding the last token one fp16 per dword (MROW = 2: a dword
+  // copy could straddle the end of the buffer range there).
   static constexpr int MROW = NG >= 2 ? NG : 2;
   static constexpr int MROW_PAIRS = NG >= 2 ? NG : 1;
   static constexpr int KB = kChunk * KL::DP;    // K code bytes per chunk
@@ -461,8 +460,14 @@ __device__ constexpr bool v_operand_in_part(int v, int part) {
 // side, the softmax) but only the V products, the partial and the merge of
 // dims [part * D / VS, (part + 1) * D / VS): less work per chunk and VS times
 // the workgroups when a launch has far fewer workgroups than the GPU has CUs.
+//
+// ALIGN: chunks start at multiples of 32 rows of the whole tensor, not of the
+// split (see aligned_chunks).  A separate instantiation: as a flag in the
+// argument block it cost every other contiguous launch 0.2-0.4 us (a load
+// ahead of the first DMA, the masked copy of the step; B = 16, HKV = 8, S = 4096,
+// 2-bit 15.6 -> 16.5).
 template <int D, int KNB, int VNB, int GS, int NW, int NSTAGE, bool PAGED, bool PT, bool KCH, int HS,
-          bool ORD, int VS, bool SMALL>
+          bool ORD, int VS, bool SMALL, bool ALIGN = false>
 __global__ void __launch_bounds__(NW * 64)
 quant_split_lds_kernel(SplitParams prm) {
   using SG = StageGeom<D, KNB, VNB, GS>;
@@ -610,16 +615,15 @@ quant_split_lds_kernel(SplitParams prm) {
       if constexpr (NG == 1) reinterpret_cast<uint32_t*>(ring + s * SG::BYTES + SG::ZERO_OFF)[i] = 0u;
     }
 
-  // Chunk k of this wave starts at token lo - head + 32 * (w + NW * k); the
-  // split's first chunk masks the `head` rows before lo (SplitParams::row_align;
-  // `early` below).
-  constexpr bool kAlign = !PAGED && !KCH && VS == 1;
-  const int first = lo - (kAlign ? (int)(((uint32_t)unit * (uint32_t)prm.S + (uint32_t)lo) &
-                                         (uint32_t)prm.row_align)
-                                 : 0);
+  // Chunk k of this wave starts at token lo + 32 * (w + NW * k).  ALIGN: at
+  // lo - head + ..., and the split's first chunk masks the `head` rows before lo
+  // (`early` below).
+  static_assert(!ALIGN || (!PAGED && !KCH && VS == 1 && NG >= 2), "aligned chunks");
+  const int first =
+      ALIGN ? lo - (int)(((uint32_t)unit * (uint32_t)prm.S + (uint32_t)lo) & (kChunk - 1u)) : lo;
   const int cb0 = first + kChunk * w;
   const int cstride = kChunk * NW;
-  static_assert(NSTAGE >= 2 && (!(PAGED || kAlign) || NSTAGE == 2), "ring depth");
+  static_assert(NSTAGE >= 2 && (!(PAGED || ALIGN) || NSTAGE == 2), "ring depth");
   // Paged: page_next is the pool page of the chunk whose DMA is issued next;
   // tab_pending the (in-flight) table entry of the chunk after that.
   int page_next = 0;
@@ -638,10 +642,10 @@ quant_split_lds_kernel(SplitParams prm) {
     static_for<NSTAGE - 1>([&](auto s) __attribute__((always_inline)) {
       constexpr int SS = decltype(s)::value;
       const int c = cb0 + SS * cstride;
-      const bool early = kAlign && c < lo;
+      const bool early = ALIGN && c < lo;
       const ChunkSrc src = chunk_src(c, 0);
       issue_chunk<D, KNB, VNB, GS, KCH>(ring + (early ? NSTAGE - 1 : SS) * SG::BYTES, src.k, src.v, src.m,
-                                        src.row, c < hi, lane, c + kChunk < hi && !early);
+                                        src.row, c < hi, lane, c + kChunk < hi);
     });
   }
 
@@ -818,7 +822,7 @@ quant_split_lds_kernel(SplitParams prm) {
   // overwrites the chunk's row with the patch, so the step never depends on
   // when the store becomes visible to its own loads.
   uint8_t* const patch = smem + NW * SM::WAVE;
-  int cb_new = -1;  // first token of the chunk this wave patches, or -1
+  int cb_new = INT_MIN;  // first token of the chunk this wave patches (ALIGN: may be before 0), or none
   int t_new = 0;    // the new token's row within that chunk
   if (prm.k_new && L - 1 >= lo && L - 1 < hi && ((L - 1 - first) / kChunk) % NW == w) {
     const int tn = L - 1;
@@ -873,7 +877,7 @@ quant_split_lds_kernel(SplitParams prm) {
   const float lscale = prm.qk_scale * __builtin_ldexpf(1.0f, 24 - eh);  // per lane (its head)
 
   // The TAIL step masks the rows past the sequence, and its `early` form, for a
-  // split's first chunk that reaches before the split (kAlign), those there too.
+  // split's first chunk that reaches before the split (ALIGN), those there too.
   // A row before the split takes a score no key reaches; it is finite, so a
   // chunk whose other scores are all -inf keeps a finite maximum.
   auto mask_row = [&](float& x, int tok, auto early) {
@@ -1349,8 +1353,8 @@ quant_split_lds_kernel(SplitParams prm) {
     int cb = cb0;
     // A first chunk that reaches before the split: a masked copy of the step, in
     // the last stage, so that the loop starts at stage 0 and carries no mask (a
-    // mask under a branch inside it cost 0.3-1.5% where no chunk takes it).
-    if constexpr (kAlign) {
+    // mask under a branch inside it cost 0.3-1.5%).
+    if constexpr (ALIGN) {
       if (cb < lo) {
         if (lo < hi)  // an empty row or split has no chunk
           step(cb, std::true_type{}, std::integral_constant<int, NSTAGE - 1>{}, pmode, part, std::true_type{});
@@ -1473,6 +1477,33 @@ inline int device_cus() {
 template <int D, int KNB, int VNB, int GS, int HS>
 constexpr bool kDimsSplit = D == 128 && KNB == VNB && GS == 32 && HS == 8;
 
+// Whether chunks start at multiples of 32 rows of the tensor.  Where S is no
+// multiple of 32, a (b, kv head) block starts inside a cache line, and chunks
+// counted from its start load pieces of one more line per tensor each (B = 32,
+// HKV = 8, D = 128, groups of 32: 4-bit at S = 16385 112.1 -> 102.4 us, 2-bit
+// 74.8 -> 69.2, 16 head columns 116.2 -> 112.2).  An aligned split has up to
+// one more chunk, and its first is masked below the split's start, so it pays
+// for splits that stream many chunks (4-bit at S = 4121 34.0 -> 31.9 us; B = 16,
+// S = 8191, 8 waves: 35.8 -> 34.9 at 2048 tokens a split, 42.8 -> 42.9 at 1024).
+// One-group rows gained nothing (2-bit S = 8190 32.6 both ways), nor did 4-wave
+// workgroups (4-bit at S = 8191 54.2 -> 54.1).  The masked rows of the first
+// split lie before the block: their offsets wrap past the 32-bit range check,
+// which needs blocks below 2^31 bytes (codes and metadata are smaller than
+// S * D), and the mask is a large negative score (a positive scale).
+//
+// The forms that have aligned kernels are those of long splits: paired tiles,
+// and one tile at a time for more than 8 query heads.  A launch small enough
+// for the dims split runs neither below 8192 tokens, so the chunks of a call do
+// not depend on whether it leaves the dims split for an order or counters.
+template <int D, int GS, bool PT, int HS>
+constexpr bool kAlignedForm = D / GS >= 2 && PT == (HS < 16);
+constexpr int kAlignMinSplit = 4096;
+
+inline bool aligned_chunks(const SplitParams& p, int D, int waves) {
+  return p.S % kChunk != 0 && p.page_size == 0 && p.split_size >= kAlignMinSplit && waves >= 8 &&
+         p.qk_scale > 0.0f && (int64_t)p.S * D < (int64_t(1) << 31);
+}
+
 template <int D, int KNB, int VNB, int GS, bool PT, int HS, bool ORD>
 void launch_quant_pto(const SplitParams& p, dim3 grid, int waves, hipStream_t st) {
   const bool paged = p.page_size > 0;
@@ -1507,6 +1538,20 @@ void launch_quant_pto(const SplitParams& p, dim3 grid, int waves, hipStream_t st
         if (wgs < 8) go(I2{}, std::true_type{});
         else go(I2{}, std::false_type{});
       }
+      return;
+    }
+  }
+  if constexpr (kAlignedForm<D, GS, PT, HS>) {
+    if (aligned_chunks(p, D, waves)) {
+      if constexpr (kTwelveWaves<D, KNB, VNB, GS, HS, PT>) {
+        if (waves == 12) {
+          quant_split_lds_kernel<D, KNB, VNB, GS, 12, kStages8, false, PT, false, HS, ORD, 1, false, true>
+              <<<grid, dim3(12 * 64), 0, st>>>(p);
+          return;
+        }
+      }
+      quant_split_lds_kernel<D, KNB, VNB, GS, 8, kStages8, false, PT, false, HS, ORD, 1, false, true>
+          <<<grid, dim3(8 * 64), 0, st>>>(p);
       return;
     }
   }
@@ -1559,9 +1604,10 @@ inline int paired_tiles_min_split(const SplitParams& p, dim3 grid, int waves) {
 
 // ===========================================================================
 // Read-ceiling probe: what the split kernel's access pattern streams with no
-// arithmetic behind it.  Same grid, waves, 32-token chunk order, two-stage
-// per-wave ring and direct-to-LDS instructions (issue_chunk) over the same
-// contiguous caches; each chunk is consumed by one LDS read per lane, so the
+// arithmetic behind it.  Same grid, waves, 32-token chunk order (counted from
+// the split's start whatever S is), two-stage per-wave ring and direct-to-LDS
+// instructions (issue_chunk) over the same contiguous caches; each chunk is
+// consumed by one LDS read per lane, so the
 // loads stay live.  The measurement counterpart, for this kernel's read
 // pattern, of a device-copy bandwidth probe.
 // ===========================================================================
