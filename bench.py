@@ -123,20 +123,25 @@ def llama_inputs(seed, B=32, HQ=32, HKV=8, S=32768, D=128):
     return q, k, v
 
 
-# The split kernel's paired-tile form runs for GQA groups of at most 8 heads
-# and splits of at least this many tokens; grids of a workgroup per compute unit
-# or more take it earlier (paired_tiles_min_split in
-# tritonkv_amd/csrc/quant_split.h), which no shape named here reaches.
-PAIRED_TILES_MIN_SPLIT = 8192
+def paired_tiles_min_split(workgroups, waves, v_nbits):
+    """Split size from which the split kernel's paired-tile form runs for GQA groups
+    of at most 8 heads (the rule of ``paired_tiles_min_split`` in
+    tritonkv_amd/csrc/quant_split.h)."""
+    from tritonkv_amd.kernels.fused_decode_attn import compute_units
+
+    cu = compute_units() or 256
+    if 4 * workgroups < 3 * cu if v_nbits == 2 else workgroups < cu:
+        return 8192
+    return 2048 if waves <= 4 else 4096
 
 
-def split_kernel_name(D, kbits, vbits, gs, waves, G, split_size, paged=False, kch=False,
+def split_kernel_name(D, kbits, vbits, gs, waves, G, split_size, workgroups, paged=False, kch=False,
                       ordered=False, vsplit=1, small_grid=False, aligned=False):
     """The demangled name (as rocprofv3 prints it) of the quantized split
     kernel instantiation that a launch with these arguments runs (``vsplit``:
     2 or 4 for the dims-split kernels of small grids, ``small_grid`` for their
     layout on fewer than 8 tuples, ``aligned`` for chunks on cache lines)."""
-    pt = not kch and G <= 8 and split_size >= PAIRED_TILES_MIN_SPLIT
+    pt = not kch and G <= 8 and split_size >= paired_tiles_min_split(workgroups, waves, vbits)
     hs = 16 if D // gs < 2 else 4 if G <= 4 else 8 if G <= 8 else 16  # head columns
     b = lambda x: "true" if x else "false"  # noqa: E731
     return (f"void tkv::quant_split_lds_kernel<{D}, {kbits}, {vbits}, {gs}, {waves}, 2, "
@@ -240,7 +245,8 @@ def fused_call(q, kq, vq, num_splits=None, split_only=False, waves=None, fused_c
         _lib.check(fn(args, torch.cuda.current_stream().cuda_stream), "fused")
     call.keep = (out, acc, mx, sm, cnt, q, kq, vq)
     call.num_splits = ns
-    call.kernel = split_kernel_name(D, kq.nbits, vq.nbits, kq.group_size, wv, HQ // HKV, size)
+    call.kernel = split_kernel_name(D, kq.nbits, vq.nbits, kq.group_size, wv, HQ // HKV, size,
+                                    B * HKV * -(-HQ // HKV // 16) * ns)
     return call
 
 
@@ -406,7 +412,7 @@ def _counter_per_dispatch(directory, kernel):
 
 def rocprof_summary(a) -> int:
     if a.kernel is None:
-        a.kernel = split_kernel_name(128, 4, 4, 32, 8, 4, 32768)
+        a.kernel = split_kernel_name(128, 4, 4, 32, 8, 4, 32768, 256)
     out = []
     out.append(a.title or f"# rocprofv3 summary -- kernel {a.kernel}..., Llama-3-8B decode step "
                f"(B=32 HQ=32 HKV=8 D=128 ctx=32768, 4-bit gs32), bench.py --quick")

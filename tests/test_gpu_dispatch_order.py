@@ -218,6 +218,8 @@ def test_equal_lengths_take_the_unragged_plan(monkeypatch, length):
 
 
 @pytest.mark.parametrize("B,HQ,HKV,S,nbits,ns", [
+    (50, 64, 8, 3000, 4, None),  # 4 waves, one split of 2048..4095 tokens on a full grid
+    (50, 32, 8, 2100, 2, None),
     (1, 12, 2, 5001, 4, 1),      # a dims-split grid whose blocks start inside a cache line
     (1, 12, 2, 9001, 2, 2),
     (4, 12, 2, 8101, 4, 1),

@@ -1588,18 +1588,23 @@ void launch_quant_pt(const SplitParams& p, dim3 grid, int waves, hipStream_t st)
 // Split sizes from which paired tiles run, for GQA groups of at most 8 query
 // heads.  They issue a third less per chunk, but build twice the q operands per
 // wave (about 1 us), and their registers let two 4-wave workgroups share a CU
-// instead of three.  Grids of about a workgroup per CU or more (B = 32 or 64,
-// HKV = 8, 4-bit groups of 32, one split):
-//   8 waves  S = 512 8.5 -> 9.2 us, 2048 18.6 -> 18.0, 4096 30.6 -> 30.1
-//   4 waves  S = 1024 18.4 -> 18.0, 4096 55.5 -> 55.2 (2-bit 43.2 -> 39.8)
-// In a dispatch order (rows of different lengths) short rows pay the longer
-// prologue: 4 waves, pieces of 2048 42.2 -> 44.4 us, of 4096 72.9 -> 71.2.
-// Smaller grids keep the threshold of 8192 tokens: equal at 4096, 5-10%
+// instead of three.  The grid, the split and the format decide, never a
+// dispatch order, whose output must not depend on it.  HKV = 8, one tile at a
+// time -> paired, us:
+//   4 waves, from 2048: B = 64 S = 2048 4-bit 31.2 -> 30.8, 2-bit 22.4 -> 22.0, groups
+//     of 128 20.6 -> 19.3, K4/V2 G = 8 26.5 -> 26.6; 4096 55.5 -> 54.8, 40.9 -> 39.5,
+//     35.9 -> 31.7, 48.6 -> 46.9
+//   8 waves, from 4096: B = 32 S = 2048 2-bit 13.5 -> 14.6, K4/V2 16.1 -> 16.4; 4096 4-bit
+//     30.6 -> 30.2, 2-bit 22.4 -> 22.0, groups of 128 21.1 -> 19.3, of 16 28.7 -> 27.4
+// On three quarters of a workgroup per CU only 2-bit values gain (B = 24, S = 4096
+// K4/V2 22.7 -> 22.4, 2-bit groups of 128 19.6 -> 18.8, but 4-bit 24.5 -> 25.1, groups
+// of 64 22.5 -> 23.1).  Otherwise 8192 tokens: equal at 4096 on small grids, 5-10%
 // slower at 512-1024, and a dims split is faster there.
-inline int paired_tiles_min_split(const SplitParams& p, dim3 grid, int waves) {
-  const unsigned long long wgs = 1ull * grid.x * grid.y * grid.z;
-  if (4 * wgs < 3ull * device_cus()) return 8192;
-  return waves <= 4 && p.order ? 4096 : 2048;
+template <int VNB>
+inline int paired_tiles_min_split(dim3 grid, int waves) {
+  const unsigned long long wgs = 1ull * grid.x * grid.y * grid.z, cus = (unsigned long long)device_cus();
+  if (VNB == 2 ? 4 * wgs < 3 * cus : wgs < cus) return 8192;
+  return waves <= 4 ? 2048 : 4096;
 }
 
 // ===========================================================================
@@ -1696,7 +1701,7 @@ void launch_quant_hs(const SplitParams& p, dim3 grid, int waves, hipStream_t st)
       return;
     }
   }
-  if (p.G <= 8 && p.split_size >= paired_tiles_min_split(p, grid, waves))
+  if (p.G <= 8 && p.split_size >= paired_tiles_min_split<VNB>(grid, waves))
     launch_quant_pt<D, KNB, VNB, GS, true, HS>(p, grid, waves, st);
   else launch_quant_pt<D, KNB, VNB, GS, false, HS>(p, grid, waves, st);
 }
