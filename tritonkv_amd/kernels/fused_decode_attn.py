@@ -156,15 +156,21 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
 
     ``fine``: the caller runs short ragged pieces in 4-wave workgroups
     (``choose_waves``), of which a CU holds two or three, so that a finer cut
-    costs little and evens out rows of different lengths (K4/V2, G = 8, in us):
+    costs little and evens out rows of different lengths.  Where the rules
+    above leave one split on half a unit to one unit per CU (or two, at exactly
+    half), a long enough history is cut into 4 workgroups per CU, in pieces
+    of at least 1024 tokens.  The fuller the grid, the longer the rows must be
+    for that to pay (HKV = 8, lengths from S/16 or S/64 to S, mean of three draws,
+    as above -> cut, us, for 4-bit G = 4 / 2-bit G = 4 / K4V2 G = 8):
 
-    * half a unit to one unit per CU: 4 workgroups per CU in pieces of at least
-      1024 tokens (24 rows of up to 32768: 111.8 at 1 split -> 84-90 at 4-8;
-      20 rows of up to 4096: 22.3 -> 20.0; 16 rows of up to 8192: 26.7 -> 24.5;
-      16 rows of up to 2048: 13.4 either way at best, so not below 4096);
-    * one to two units per CU and 65536 tokens or more: pieces of 8192-16384
-      tokens (32 rows of up to 65536: 174 at 2 splits -> 172 at 6, 2-bit 143 ->
-      133, 4-bit 205 -> 201).
+    * 17 rows of up to 4096: 20.5 -> 17.1, 18.8 -> 15.8, 21.0 -> 17.8;
+    * 24 rows: 4096 21.4 -> 22.3, 19.2 -> 19.4, 21.2 -> 21.7 (not cut); 8192
+      35.2 -> 31.6, 29.9 -> 25.1, 33.2 -> 29.0;
+    * 28 rows: 8192 38.8 -> 43.4, 31.3 -> 30.1, 35.7 -> 41.3 (not cut); 16384
+      65.3 -> 55.6, 53.8 -> 42.2, 59.9 -> 49.4;
+    * 16 rows: 8192 25.7 -> 26.1, 22.5 -> 22.2, 24.8 -> 25.9 and 16384 42.2 ->
+      44.4, 35.1 -> 31.0, 38.4 -> 41.9 (not cut); 32768 72.4 -> 65.1, 58.8 ->
+      46.1, 65.2 -> 59.0.
 
     Returned in units of ``block_n`` blocks so the reference's tightening
     applies unchanged.
@@ -176,10 +182,14 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
     if units >= cu:
         if not ragged or S < 16384:
             return 1
-        piece = 32768 if units >= 2 * cu or S < 65536 or not fine else 10922
-        return min(max(2, S // piece), _cdiv(S, block_n))
-    if ragged and fine and 2 * units >= cu and S >= 4096:
-        return max(1, min(4 * cu // units, S // 1024, _cdiv(S, block_n)))
+        return min(max(2, S // 32768), _cdiv(S, block_n))
+    if ragged and fine and 2 * units >= cu:
+        if 2 * units == cu:
+            least = 32768
+        else:
+            least = 4096 if 8 * units <= 5 * cu else 8192 if 4 * units <= 3 * cu else 16384
+        if S >= least:
+            return max(1, min(4 * cu // units, S // 1024, _cdiv(S, block_n)))
     workgroups = min(cu, max(32, units * S // tokens_per_workgroup))
     want = max(1, workgroups // units)
     max_splits = max(1, S // max(tokens_per_workgroup // 4, block_n))
