@@ -254,3 +254,33 @@ def test_paged_step_replays_in_a_graph():
         for a, b in zip((kp.packed, kp.scale, kp.zero, vp.packed, vp.scale, vp.zero),
                         (*kp2, *vp2)):
             assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("B,S,kbits,vbits,G,ns,order", [
+    (50, 4160, 4, 4, 4, None, True), (50, 8320, 4, 4, 4, 1, True), (64, 4160, 4, 2, 8, None, False),
+    (24, 2048, 4, 4, 4, 4, False), (20, 3072, 2, 2, 4, 3, None),
+])
+def test_repeated_paged_calls_give_the_same_bits(B, S, kbits, vbits, G, ns, order):
+    """Every wave waits for all of its last chunk, whatever the number of chunks
+    before it: rows of every length, many calls, each equal to the contiguous one."""
+    from tritonkv_amd.kernels import fused_decode_attention
+    from tritonkv_amd.paged import paged_decode_attention
+    from tritonkv_amd.quantize import quantize_groupwise
+
+    print(f"repeated paged calls B={B} S={S} K{kbits}V{vbits} G={G} ns={ns}", flush=True)
+    HKV, page = 8, 64
+    g = torch.Generator(device=DEV).manual_seed(S + B)
+    q = torch.randn(B, HKV * G, 128, device=DEV, generator=g, dtype=torch.float16)
+    x = torch.randn(B, HKV, S, 128, device=DEV, generator=g, dtype=torch.float16)
+    kq, vq = quantize_groupwise(x, kbits, 32), quantize_groupwise(x.flip(2), vbits, 32)
+    num_pages = B * S // page + 3
+    table = _random_table(B, S // page, num_pages, seed=B)
+    kp, vp = (_scatter_to_pool(t, table, num_pages, page) for t in (kq, vq))
+    lens = torch.randint(1, S + 1, (B,), generator=torch.Generator().manual_seed(S)).to(torch.int32).to(DEV)
+    kw = dict(num_splits=ns, allow_mixed_bits=True, dispatch_order=order)
+    want = fused_decode_attention(q, kq, vq, seq_lens=lens, **kw)
+    ws = {}
+    wrong = torch.zeros((), dtype=torch.int64, device=DEV)
+    for _ in range(200):
+        wrong += (paged_decode_attention(q, kp, vp, table, lens, _workspace=ws, **kw) != want).sum()
+    assert int(wrong) == 0

@@ -635,6 +635,7 @@ quant_split_lds_kernel(SplitParams prm) {
     const ChunkSrc src = chunk_src(cb0, page0);
     issue_chunk<D, KNB, VNB, GS, KCH>(ring, src.k, src.v, src.m, src.row, cb0 < hi, lane,
                                       cb0 + kChunk < hi);
+    asm volatile("" ::: "memory");  // behind the DMA (see the wait in step)
     tab_pending = tab_entry(cb0 + 2 * cstride);
   } else {
     // the first NSTAGE - 1 chunks into stages 0 .. NSTAGE - 2; a chunk that
@@ -936,12 +937,22 @@ quant_split_lds_kernel(SplitParams prm) {
       issue_chunk<D, KNB, VNB, GS, KCH>(ring + ((SK + NSTAGE - 1) % NSTAGE) * SG::BYTES, src.k, src.v,
                                    src.m, src.row, valid, lane, cn + kChunk < hi);
     }
-    // Paged: one more vector load in flight, behind the DMA just issued.
+    // Paged: one more vector load in flight, behind the DMA just issued -- but
+    // not in the TAIL step, after which no chunk follows.  The wait may count a
+    // table load only where the code keeps it: the step ahead of the TAIL and the
+    // TAIL itself have no use for theirs, the compiler drops both, and a wait
+    // that counted one there returned with the last DMA instruction of the TAIL's
+    // own chunk (its V zero points) still in flight.  Any other step's chunk was
+    // issued ahead of the table load of the page after it, which is used.
+    constexpr bool TAB = PAGED && !TAIL;
     uint32_t tab_new = 0;
-    if constexpr (PAGED) tab_new = tab_entry(cb + 3 * cstride);
-    wait_vmcnt<(NSTAGE - 1) * NI + (PAGED ? 1 : 0)>();
+    if constexpr (TAB) {
+      asm volatile("" ::: "memory");  // the load stays behind the DMA
+      tab_new = tab_entry(cb + 3 * cstride);
+    }
+    wait_vmcnt<(NSTAGE - 1) * NI + (TAB ? 1 : 0)>();
     asm volatile("" ::: "memory");  // no LDS read of this stage above the wait
-    if constexpr (PAGED) {  // retired with the wait above: issued a step ago
+    if constexpr (TAB) {
       page_next = to_page(tab_pending);
       tab_pending = tab_new;
     }
