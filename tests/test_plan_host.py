@@ -26,3 +26,49 @@ def test_ragged_batches_are_cut_where_that_was_measured_to_pay(B, S, splits):
     # the fp16 control and per-channel keys keep the even cut
     even = plan_splits(S, 64, None, B, 8, 4, ragged=True, fine=False)[1]
     assert even == {16: 2}.get(B, 1) if B < 32 else even == splits
+
+
+FP16, K4, K2, K42 = (16, 16, 0), (4, 4, 32), (2, 2, 32), (4, 2, 32)
+ONE4, ONE2 = (4, 4, 128), (2, 2, 128)
+
+
+@pytest.mark.parametrize("fmt,D,B,S,ns,ragged,waves", [
+    (K4, 128, 47, 1024, 1, False, 8), (K4, 128, 48, 1024, 1, False, 4), (K4, 128, 64, 32768, 1, False, 4),
+    (K2, 128, 64, 32768, 1, False, 4), (K2, 128, 64, 40960, 1, False, 12),
+    (ONE4, 128, 64, 32768, 1, False, 4),
+    (FP16, 128, 64, 8192, 1, False, 4), (FP16, 128, 128, 16384, 1, False, 8), (FP16, 64, 64, 1024, 1, False, 8),
+    (K4, 64, 64, 16384, 1, False, 4), (K2, 64, 64, 4096, 1, False, 8), (K2, 64, 128, 4096, 1, False, 4),
+    (K42, 64, 64, 16384, 1, False, 8),
+    (K4, 128, 64, 3072, 1, True, 4), (K4, 128, 64, 4096, 1, True, 8), (K4, 128, 128, 4096, 1, True, 4),
+    (K4, 128, 24, 4096, 4, True, 4), (K4, 128, 128, 8192, 1, True, 4), (K4, 128, 64, 16384, 2, True, 8),
+    (K2, 128, 64, 16384, 2, True, 4), (K4, 128, 64, 32768, 3, True, 4),
+    (ONE4, 128, 128, 8192, 1, True, 4), (ONE4, 128, 64, 16384, 2, True, 12), (ONE4, 128, 96, 16384, 2, True, 4),
+    (ONE4, 128, 64, 32768, 3, True, 12), (ONE2, 128, 64, 32768, 2, True, 4),
+    (FP16, 128, 64, 512, 1, True, 4), (FP16, 128, 64, 1024, 1, True, 8), (FP16, 64, 64, 512, 1, True, 8),
+    (K2, 64, 64, 2048, 1, True, 8), (K2, 64, 128, 2048, 1, True, 4), (K4, 64, 128, 8192, 1, True, 8),
+])
+def test_four_waves_run_where_they_were_measured_to_pay(fmt, D, B, S, ns, ragged, waves):
+    from tritonkv_amd.kernels.fused_decode_attn import choose_waves
+
+    k, v, gs = fmt
+    assert choose_waves(B, 8, 4, S, ns, D=D, k_nbits=k, v_nbits=v, group_size=gs, ragged=ragged) == waves
+
+
+def test_per_channel_keys_keep_larger_workgroups_on_long_pieces():
+    from tritonkv_amd.kernels.fused_decode_attn import choose_waves
+
+    kw = dict(D=128, k_nbits=2, v_nbits=2, group_size=32, ragged=True)
+    assert choose_waves(64, 8, 4, 16384, 2, **kw) == 4
+    assert choose_waves(64, 8, 4, 16384, 2, per_channel=True, **kw) == 12
+    assert choose_waves(128, 8, 4, 4096, 1, per_channel=True, **kw) == 4
+    assert choose_waves(128, 8, 4, 8192, 1, per_channel=True, **kw) == 12
+    kw["ragged"] = False
+    assert choose_waves(64, 8, 4, 16384, 1, per_channel=True, **kw) == 4
+    assert choose_waves(64, 8, 4, 24576, 1, per_channel=True, **kw) == 12
+
+
+def test_page_pools_of_head_dim_64_keep_larger_workgroups():
+    from tritonkv_amd.kernels.fused_decode_attn import choose_waves
+
+    kw = dict(D=64, k_nbits=4, v_nbits=4, group_size=64, paged=True)
+    assert [choose_waves(B, 8, G, 4096, 1, **kw) for B, G in ((64, 4), (128, 4), (64, 16))] == [8, 4, 4]

@@ -208,7 +208,7 @@ def channel_decode_attention(
         v_nbits=vq.nbits, group_size=vq.group_size, sm_scale=float(sm_scale),
         split_size=split_size, num_splits=num_splits, counters=None,
         waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, k_nbits=ck.nbits,
-                           v_nbits=vq.nbits, group_size=vq.group_size, ragged=ragged),
+                           v_nbits=vq.nbits, group_size=vq.group_size, ragged=ragged, per_channel=True),
         key_block=BLOCK)
     rc = _lib.launch(q.device, "tkv_channel_decode_attention", args, kr.data_ptr(), vr.data_ptr(),
                      _lib.ptr(rlens), R)

@@ -105,7 +105,7 @@ def fp16_decode_attention(
         acc=_lib.ptr(acc), maxs=_lib.ptr(maxs), sums=_lib.ptr(sums), out=out.data_ptr(),
         B=B, HQ=HQ, HKV=HKV, S=S, D=D, k_nbits=16, v_nbits=16, group_size=D,
         sm_scale=float(sm_scale), split_size=split_size, num_splits=num_splits,
-        counters=None, waves=choose_waves(B, HKV, group, split_size, num_splits, ragged=ragged))
+        counters=None, waves=choose_waves(B, HKV, group, split_size, num_splits, D=D, ragged=ragged))
     rc = _lib.launch(q.device, "tkv_fp16_decode_attention", args)
     _lib.check(rc, "fp16_decode_attention")
     # k / v are read in place; a converted copy (not fp16, not contiguous) is not kept

@@ -216,35 +216,73 @@ def twelve_wave_format(D: int, G: int, k_nbits: int, v_nbits: int, group_size: i
         (k_nbits == v_nbits and k_nbits in (2, 4) and group_size == 128)
 
 
+def _four_waves_pay(wgs: int, cu: int, split_size: int, num_splits: int, G: int, D: int,
+                    k_nbits: int, v_nbits: int, group_size: int, twelve: bool, paged: bool,
+                    ragged: bool, per_channel: bool) -> bool:
+    """Whether a grid of at least one and a half workgroups per compute unit runs
+    4 waves.  A CU then holds two or three workgroups at once, and one streams
+    while another builds its q operands or merges; an 8-wave workgroup fills a
+    CU's LDS or registers alone.  Figures: HKV = 8, the 8 or 12 waves it would
+    run otherwise -> 4, us.
+
+    Equal lengths, D = 128, G = 4, 64 rows: 4-bit ctx 1024 21.8 -> 18.1, 4096
+    58.5 -> 55.6, 16384 203 -> 199, 32768 396 -> 393; 2-bit 4096 43.6 -> 40.8, 32768
+    268 -> 265; groups of 128 4-bit 1024 19.0 -> 15.8, 32768 348 -> 343, 2-bit 223 ->
+    224; per-channel 2-bit 4096 55.9 -> 50.2, 16384 160.7 -> 161.5, 24576 235 ->
+    238.  The fp16 control: 1024 44.7 -> 43.3, 8192 306 -> 303, 128 rows of 16384
+    1223 -> 1235.  D = 64: 4-bit 4096 27.6 -> 26.4, 32768 191 -> 183; 2-bit, and page pools
+    below 9 query heads, only from four workgroups per CU (64 rows of 4096 22.0 ->
+    23.3, 128 rows 41.5 -> 39.2; paged 4-bit 29.6 -> 39.8, 128 rows of 2048 34.4 -> 29.2).
+
+    Rows of different lengths (mean of three to five draws): fewer, larger
+    workgroups balance better unless the pieces are short or many.  One piece a
+    row: 64 rows of up to 3072 4-bit 33.7 -> 30.6, 2-bit 28.9 -> 24.6, but 48 rows of up
+    to 4096 34.5 -> 36.1, 28.4 -> 29.3; rows cut on purpose have mostly full pieces
+    (32 rows of up to 16384 in 4: 77.5 -> 73.2).  Four workgroups per CU: 128 rows
+    of up to 8192 132 -> 129, 2-bit 99 -> 90, groups of 128 4-bit 117 -> 113, but
+    per-channel 4-bit 145 -> 151 (of up to 4096 93 -> 89); 64 rows of up to 32768 in
+    pieces of 16384 4-bit 239 -> 243, 2-bit 168 -> 158, per-channel 2-bit 210 -> 214,
+    groups of 128 4-bit 207 -> 212; six, 96 rows of them 353 -> 348, 250 -> 235, 302 ->
+    301, 310 -> 309, and in pieces of 32768 654 -> 657, 449 -> 439, 554 -> 550, 572 ->
+    587.  The fp16 control: 64 rows of up to 512 20.1 -> 18.4, 1024 34.2 -> 35.1, 16384
+    437 -> 494.  D = 64: 128 rows of up to 4096 2-bit 35.8 -> 33.5, 64 rows 20.4 -> 22.0."""
+    many = wgs >= 4 * cu
+    if k_nbits == 16:
+        return D == 128 and split_size <= (512 if ragged else 8192)
+    if D == 64:
+        if ragged:
+            return many and split_size <= 4096
+        return (many and split_size <= 8192) or (
+            min(k_nbits, v_nbits) == 4 and split_size <= 32768 and not (paged and G <= 8))
+    if not ragged:
+        return split_size <= (16384 if twelve and per_channel else 32768)
+    if split_size <= (4096 if num_splits > 1 else 3072):
+        return True
+    two_bit = k_nbits == 2 and v_nbits == 2
+    if not many or split_size > 32768:
+        return False
+    if wgs >= 6 * cu and split_size > 8192:
+        return two_bit or group_size != D or split_size <= 16384
+    return split_size <= (4096 if per_channel else 8192) or (two_bit and not per_channel)
+
+
 def choose_waves(B: int, HKV: int, G: int, split_size: int, num_splits: int = 0, *,
                  D: int = 128, k_nbits: int = 16, v_nbits: int = 16, group_size: int = 0,
-                 paged: bool = False, ragged: bool = False) -> int:
-    """Waves per workgroup.
-
-    4 when the grid holds at least one and a half workgroups per compute unit
-    and none streams more than 32768 tokens: a CU then holds two or three of
-    them at once, and one streams while another builds its q operands or merges
-    (an 8-wave workgroup fills a CU's LDS or registers alone).  HKV = 8, G = 4,
-    8 or 12 waves -> 4, us: B = 64 4-bit ctx 1024 21.8 -> 18.0, 4096 58.9 ->
-    55.2, 16384 205.3 -> 201.5; 2-bit ctx 4096 45.9 -> 39.8, 16384 142 -> 134;
-    B = 128 ctx 1024 42.7 -> 33.3; at one workgroup per CU 2-bit ctx 4096
-    22.7 -> 24.6.  With rows of different lengths (``ragged``) fewer, larger
-    workgroups balance better until there are many pieces or they are short:
-    4 waves from four workgroups per CU (64 rows of up to 131072, 4 splits
-    647 -> 630) or for pieces of at most 4096 tokens (64 rows of up to 1024
-    21.2 -> 14.3, 4096 41.4 -> 40.6, but 8192 63.2 -> 69.3).
-
-    Otherwise 12 for the formats of ``twelve_wave_format`` when a
-    workgroup streams at least ``TWELVE_WAVES_MIN_SPLIT`` tokens; else 8 when
+                 paged: bool = False, ragged: bool = False, per_channel: bool = False) -> int:
+    """Waves per workgroup: 4 on grids of at least one and a half workgroups per
+    compute unit where ``_four_waves_pay``; else 12 for the formats of
+    ``twelve_wave_format`` when a workgroup streams at least
+    ``TWELVE_WAVES_MIN_SPLIT`` tokens; else 8 when
     it streams the whole history or at least 512 tokens (two 32-token chunks
     per wave, so each wave overlaps a load with compute); else 4.  The default
-    format (16-bit) is the fp16 control's."""
+    format (16-bit) is the fp16 control's; ``ragged``: rows of different
+    lengths; ``per_channel``: per-channel keys."""
     wgs, cu = B * HKV * _cdiv(G, 16) * num_splits, compute_units() or 256
-    if 2 * wgs >= 3 * cu and split_size <= 32768 and \
-            (not ragged or wgs >= 4 * cu or split_size <= 4096):
+    twelve = twelve_wave_format(D, G, k_nbits, v_nbits, group_size, paged)
+    if 2 * wgs >= 3 * cu and _four_waves_pay(wgs, cu, split_size, num_splits, G, D, k_nbits, v_nbits,
+                                             group_size, twelve, paged, ragged, per_channel):
         return 4
-    if split_size >= TWELVE_WAVES_MIN_SPLIT and \
-            twelve_wave_format(D, G, k_nbits, v_nbits, group_size, paged):
+    if split_size >= TWELVE_WAVES_MIN_SPLIT and twelve:
         return 12
     return 8 if num_splits == 1 or split_size >= 512 else 4
 
