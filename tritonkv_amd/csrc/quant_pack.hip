@@ -85,6 +85,12 @@ struct WideRow {
   static constexpr int P = 8 / NB, DP = D / P, NG = D / GS, QMAX = (1 << NB) - 1, E = 8;
   static constexpr int LPR = DP / E, RPS = 64 / LPR;  // lanes per row, rows per wave and step
   static constexpr int NV = F32 ? 2 : 1;              // 16-byte loads per run of E values
+  // Rows are read once, but where several of a wave's load instructions take
+  // pieces of the same cache line, a non-temporal line is gone before the last of
+  // them (524288 rows, plain -> non-temporal loads, us: D = 64 2-bit fp16 15.6 ->
+  // 21.5, fp32 26.7 -> 40.6, 4-bit fp16 17.4 -> 18.6; D = 128 2-bit fp32 54.2 -> 54.7).
+  // fp16 rows of 128 dims gain: 4-bit 31.8 -> 31.3, 2-bit 31.3 -> 30.3.
+  static constexpr bool kNonTemporal = D == 128 && !F32;
   static_assert(DP % E == 0 && LPR >= 2 && LPR <= 16, "row shape");
   static_assert(GS > DP ? GS % DP == 0 : GS % E == 0, "group shape");
 
@@ -100,11 +106,11 @@ struct WideRow {
     for (int p = 0; p < P; ++p)
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
-        // read once: non-temporal (35.2 -> 31.5 us for the 4-bit rows below)
         const int64_t e = off + p * DP + c * E;
         const u4* v = F32 ? reinterpret_cast<const u4*>(static_cast<const float*>(x) + e)
                           : reinterpret_cast<const u4*>(static_cast<const _Float16*>(x) + e);
-        raw[p][k] = __builtin_nontemporal_load(v + k);
+        if constexpr (kNonTemporal) raw[p][k] = __builtin_nontemporal_load(v + k);
+        else raw[p][k] = v[k];
       }
   }
 
