@@ -69,3 +69,20 @@ def test_several_steps_per_wave_match_the_oracle_bitwise(nbits, gs, dtype):
     assert np.array_equal(qt.packed.cpu().numpy(), ref.packed)
     assert np.array_equal(qt.scale.cpu().numpy().view(np.uint16), ref.scale.view(np.uint16))
     assert np.array_equal(qt.zero.cpu().numpy().view(np.uint16), ref.zero.view(np.uint16))
+
+
+@pytest.mark.parametrize("nbits,gs,D", [(4, 32, 128), (2, 64, 128), (2, 32, 64)])
+@pytest.mark.parametrize("B,HKV,N", [(2, 3, 15), (2, 3, 31), (2, 3, 57), (2, 3, 65),  # small workgroups
+                                     (512, 4, 32), (512, 4, 33), (256, 4, 64), (256, 4, 96),
+                                     (256, 4, 111), (256, 4, 112), (256, 4, 129), (128, 4, 256)])
+def test_prompts_on_both_sides_of_the_fill_rule(nbits, gs, D, B, HKV, N):
+    """By head or all heads together: the same rows as one long run of them."""
+    from tritonkv_amd.quantize import append_kv, empty_cache, quantize_groupwise
+
+    print(f"fill rule {nbits}-bit gs{gs} D={D} B={B} HKV={HKV} N={N}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(B, HKV, N, D, device=DEV, generator=g, dtype=torch.float16)
+    got = append_kv(empty_cache(B, HKV, N, D, nbits, gs, DEV), x)
+    want = quantize_groupwise(x.view(1, 1, -1, D), nbits, gs)
+    for a, b in ((got.packed, want.packed), (got.scale, want.scale), (got.zero, want.zero)):
+        assert torch.equal(a.view(-1, a.shape[-1]), b.view(-1, b.shape[-1]))

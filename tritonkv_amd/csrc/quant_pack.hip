@@ -274,13 +274,13 @@ quantize_pack_wide_kernel(const void* __restrict__ x, int rows, int HKV, int N,
 // running together read neighbouring memory; y is the batch row.
 // Requires x 16-byte, its strides 16-byte multiples, packed 8-byte and
 // scale / zero 4-byte aligned.
-template <int D, int NB, int GS, bool F32, int STEPS>
+template <int D, int NB, int GS, int STEPS>
 __global__ void __launch_bounds__(256)
 quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
                        const int32_t* __restrict__ positions, int start, int S_cap,
                        uint8_t* __restrict__ packed, uint16_t* __restrict__ scale,
                        uint16_t* __restrict__ zero) {
-  using W = WideRow<D, NB, GS, F32>;
+  using W = WideRow<D, NB, GS, false>;
   constexpr int P = W::P, DP = W::DP, NG = W::NG, RPS = W::RPS, ROWS = STEPS * RPS;
   __shared__ __attribute__((aligned(16))) uint32_t meta_lds[4][ROWS * NG];
 
@@ -795,10 +795,6 @@ unpack_v_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__
   }
 }
 
-// Tokens per head from which a workgroup takes tokens of one head only
-// (quantize_tokens_kernel).  Below it most of a workgroup's rows would be
-// empty, and the rows of all heads are run together (quantize_pack_wide_kernel).
-constexpr int kTokensMinN = 32;
 // Rows from which a wave takes several steps of rows: fewer rows run one step
 // per wave, at most eight waves for each of the chip's 1024 SIMDs.
 constexpr int64_t kBulkRows = 65536;
@@ -810,29 +806,51 @@ static constexpr int quantize_steps(bool f32, bool bulk) {
   return bulk && 8 / per > 0 ? 8 / per : 1;
 }
 
+// fp16 tokens a workgroup of quantize_tokens_kernel takes.
+template <int D, int NB, int GS>
+static constexpr int tokens_per_wg(bool bulk) {
+  return 4 * WideRow<D, NB, GS, false>::RPS * quantize_steps<NB>(false, bulk);
+}
+
+// Whether N tokens a head fill such workgroups well enough.  All tokens of one
+// belong to one head, so a head's last workgroup is partly empty, where
+// quantize_pack_wide_kernel runs the rows of all heads together (8192 heads, 128
+// tokens a workgroup, 4-bit, us, all heads together -> by head: N = 33 21.7 -> 29.5,
+// 64 34.8 -> 32.5, 80 41.4 -> 41.5, 96 48.6 -> 44.8, 100 50.4 -> 51.5, 128 63.4 -> 57.2,
+// 129 64.0 -> 88.9, 200 97.3 -> 99.2, 257 127.9 -> 139.6, 300 149 -> 159): seven eighths
+// full, or one workgroup a head at least half full of whole waves.  4-bit rows of
+// 128 dims whose input the last-level cache holds (256 MB; a quarter of it where a
+// head has one workgroup) gain earlier (2048 heads: N = 65 13.8 -> 12.4, 80 14.6 -> 13.2,
+// 100 18.0 -> 16.0, 129 21.4 -> 27.0, 160 24.7 -> 27.7, 200 29.3 -> 28.8, 257 34.9 -> 34.1, 300
+// 39.5 -> 37.2; 256 heads, 257 9.0 -> 7.9; 8192 heads, 65 35.2 -> 40.0), 2-bit ones do
+// not (100 15.2 -> 16.0, 300 36.6 -> 37.8).
+template <int D, int NB, int GS>
+static bool tokens_fill_wgs(int64_t rows, int N, bool bulk) {
+  const int per_wg = tokens_per_wg<D, NB, GS>(bulk);
+  constexpr bool early = D == 128 && NB == 4;
+  if (N < per_wg) return 2 * N >= per_wg && ((early && rows <= 1 << 18) || N % (per_wg / 4) == 0);
+  const int64_t room = ((int64_t)N + per_wg - 1) / per_wg * per_wg;
+  return early && rows <= 1 << 20 ? 3 * (int64_t)N >= 2 * room : 8 * (int64_t)N >= 7 * room;
+}
+
 // quantize_tokens_kernel for what it takes; false (nothing launched) otherwise.
 template <int D, int NB, int GS>
-static bool launch_tokens(const TokenSource& src, bool f32, int B, int HKV, int N,
+static bool launch_tokens(const TokenSource& src, bool bulk, int B, int HKV, int N,
                           const int32_t* pos, int start, int S_cap, uint8_t* pk, uint16_t* sc,
                           uint16_t* zr, hipStream_t st) {
-  const int es = f32 ? 4 : 2;
-  const uintptr_t align = (uintptr_t)src.x | (uintptr_t)(src.sb * es) | (uintptr_t)(src.sh * es) |
-                          (uintptr_t)(src.st * es);
+  const uintptr_t align = (uintptr_t)src.x | (uintptr_t)(src.sb * 2) | (uintptr_t)(src.sh * 2) |
+                          (uintptr_t)(src.st * 2);
   if ((align & 15) || ((uintptr_t)pk & 7) || (((uintptr_t)sc | (uintptr_t)zr) & 3)) return false;
-  const bool bulk = (int64_t)B * HKV * N >= kBulkRows;
-  const int per_wg = 4 * WideRow<D, NB, GS, false>::RPS * quantize_steps<NB>(f32, bulk);
+  const int per_wg = tokens_per_wg<D, NB, GS>(bulk);
   const int64_t tiles = ((int64_t)N + per_wg - 1) / per_wg;
-  if (N < kTokensMinN || B > 65535 || tiles * HKV > INT32_MAX / 256) return false;
+  if (B > 65535 || tiles * HKV > INT32_MAX / 256) return false;
   const dim3 grid((unsigned)(tiles * HKV), (unsigned)B);
-#define TKV_TOKENS(F, BK)                                                                       \
-  quantize_tokens_kernel<D, NB, GS, F, quantize_steps<NB>(F, BK)><<<grid, 256, 0, st>>>(        \
-      src, HKV, N, (int)tiles, pos, start, S_cap, pk, sc, zr)
-  if (f32) {
-    if (bulk) TKV_TOKENS(true, true); else TKV_TOKENS(true, false);
-  } else {
-    if (bulk) TKV_TOKENS(false, true); else TKV_TOKENS(false, false);
-  }
-#undef TKV_TOKENS
+  if (bulk)
+    quantize_tokens_kernel<D, NB, GS, quantize_steps<NB>(false, true)><<<grid, 256, 0, st>>>(
+        src, HKV, N, (int)tiles, pos, start, S_cap, pk, sc, zr);
+  else
+    quantize_tokens_kernel<D, NB, GS, quantize_steps<NB>(false, false)><<<grid, 256, 0, st>>>(
+        src, HKV, N, (int)tiles, pos, start, S_cap, pk, sc, zr);
   return true;
 }
 
@@ -840,12 +858,14 @@ template <int D, int NB, int GS>
 static void launch_quantize(const TokenSource& src, bool f32, int B, int HKV, int N,
                             const int32_t* pos, int S_cap, PageMap pm, uint8_t* pk, uint16_t* sc,
                             uint16_t* zr, hipStream_t st) {
-  if (pm.page_size == 0 && launch_tokens<D, NB, GS>(src, f32, B, HKV, N, pos, 0, S_cap, pk, sc, zr, st))
-    return;
+  // fp32 rows gain nothing from it (524288 rows of 128, 4-bit 56.1 -> 56.2 us, 2-bit 53.5 -> 54.2)
   const int64_t rows = (int64_t)B * HKV * N;
+  const bool bulk = rows >= kBulkRows;
+  if (!f32 && pm.page_size == 0 && tokens_fill_wgs<D, NB, GS>(rows, N, bulk) &&
+      launch_tokens<D, NB, GS>(src, bulk, B, HKV, N, pos, 0, S_cap, pk, sc, zr, st))
+    return;
   const bool wide = !((uintptr_t)src.x & 15) && !((uintptr_t)pk & 7);
   if (wide && rows <= INT32_MAX) {
-    const bool bulk = rows >= kBulkRows;
     const int per_wg = 4 * WideRow<D, NB, GS, false>::RPS * quantize_steps<NB>(f32, bulk);
     const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
     const int r = (int)rows;
@@ -1084,7 +1104,7 @@ extern "C" int tkv_channel_extend(const void* k, const int64_t* k_strides, const
   if (whole) {
     bool done = false;
 #define TKV_VT(Dv, NBv, GSv) \
-  done = launch_tokens<Dv, NBv, GSv>(vs, false, B, HKV, whole, nullptr, start, S_cap, v_packed, v_scale, v_zero, st)
+  done = launch_tokens<Dv, NBv, GSv>(vs, (int64_t)B * HKV * whole >= kBulkRows, B, HKV, whole, nullptr, start, S_cap, v_packed, v_scale, v_zero, st)
     TKV_DISPATCH_DNG(D, v_nbits, group_size, TKV_VT);
 #undef TKV_VT
     if (!done) return TKV_EINVAL;
