@@ -125,3 +125,26 @@ def test_another_stream_and_a_side_thread():
     t = threading.Thread(target=work)
     t.start(), t.join()
     assert torch.equal(got[0], want)
+
+
+def test_everything_runs_without_the_native_module(monkeypatch):
+    """The C ABI is all the kernels need; calls are then checked in full each time."""
+    import sys
+
+    from tritonkv_amd import _lib
+    from tritonkv_amd.kernels import fused_decode_attention
+    from tritonkv_amd.quantize import dequantize_groupwise, quantize_groupwise
+
+    q, k, _, kq, vq = make_case(1, 8, 2, 128, 600, 4, 32, seed=8)
+    want = fused_decode_attention(q, kq, vq), dequantize_groupwise(kq)
+    monkeypatch.setattr(_lib, "_HOST", None)
+    monkeypatch.setattr(_lib, "_HOST_SOUGHT", False)
+    monkeypatch.delattr("tritonkv_amd._hostcall", raising=False)
+    monkeypatch.setitem(sys.modules, "tritonkv_amd._hostcall", None)
+    monkeypatch.setattr(_lib, "_LIB", None)
+    ws = {}
+    with pytest.warns(RuntimeWarning, match="_hostcall"):
+        again = quantize_groupwise(k, 4, 32)
+    for _ in range(2):
+        assert torch.equal(fused_decode_attention(q, again, vq, _workspace=ws), want[0])
+    assert "call" not in ws and torch.equal(dequantize_groupwise(again), want[1])

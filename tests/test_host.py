@@ -489,3 +489,15 @@ def test_prepared_call_key_tracks_what_the_argument_block_depends_on():
     ws = {"call": Prep()}
     assert _prepared(ws, ("a", 1)) is ws["call"]
     assert _prepared(ws, ("a", 2)) is None
+
+
+def test_the_library_loads_without_the_native_module(monkeypatch):
+    import sys
+
+    from tritonkv_amd import _lib
+
+    monkeypatch.setattr(_lib, "_LIB", None)
+    monkeypatch.setattr(_lib, "_LOAD_ERROR", None)
+    monkeypatch.delattr("tritonkv_amd._hostcall", raising=False)
+    monkeypatch.setitem(sys.modules, "tritonkv_amd._hostcall", None)
+    assert _lib.load().tkv_abi_version() >= 1 and _lib.load_error() is None

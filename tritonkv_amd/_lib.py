@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import torch  # noqa: F401  (must be imported before the library, see above)
 
@@ -120,13 +121,14 @@ SIGNATURES = {
 
 _LIB = None
 _HOST = None
+_HOST_SOUGHT = False
 _ADDRESSES: dict = {}
 _LOAD_ERROR: str | None = None
 
 
 def load():
     """Load the library (once).  Raises RuntimeError if it is absent or broken."""
-    global _LIB, _HOST, _LOAD_ERROR
+    global _LIB, _LOAD_ERROR
     if _LIB is not None:
         return _LIB
     if not os.path.exists(LIB_PATH):
@@ -142,20 +144,23 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = restype
-    try:
-        from . import _hostcall
-    except ImportError as exc:
-        _LOAD_ERROR = f"tritonkv_amd/_hostcall.so: {exc}; run `python -m tritonkv_amd.build`"
-        raise RuntimeError(_LOAD_ERROR) from exc
-    _HOST = _hostcall
     _LIB = lib
     return lib
 
 
 def host():
-    """The CPython module of repeated calls (``csrc/host_call.cpp``)."""
-    if _HOST is None:
-        load()
+    """The CPython module of repeated calls (``csrc/host_call.cpp``), or None
+    (with one warning) where it is absent or was built against another torch:
+    the library needs only its C ABI, so every call then takes the full path."""
+    global _HOST, _HOST_SOUGHT
+    if not _HOST_SOUGHT:
+        try:
+            from . import _hostcall
+            _HOST = _hostcall
+        except ImportError as exc:
+            warnings.warn(f"tritonkv_amd/_hostcall.so: {exc}; repeated calls are checked in full "
+                          "(run `python -m tritonkv_amd.build`)", RuntimeWarning, stacklevel=2)
+        _HOST_SOUGHT = True
     return _HOST
 
 
@@ -195,7 +200,8 @@ def address(name: str) -> int:
 def launch(device: torch.device, name: str, *args) -> int:
     """The status of library call ``name`` with ``args`` on the device's current stream."""
     fn = getattr(load(), name)
-    stream = _HOST.raw_stream(device.index)
+    module = _HOST if _HOST_SOUGHT else host()
+    stream = module.raw_stream(device.index) if module is not None else None
     if stream is not None:
         return fn(*args, stream)
     with torch.cuda.device(device):

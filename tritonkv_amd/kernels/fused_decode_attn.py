@@ -499,7 +499,10 @@ _OUT_OFFSET, _Q_OFFSET, _K_NEW_OFFSET, _V_NEW_OFFSET = (
 def _keep_call(ws, key, args, entry, what, out, buffers, q, caches, lens, new=(None, None),
                window=None):
     """Put a call that just ran into the workspace for reuse, if every tensor
-    was used as it was passed (contiguous, plain storage)."""
+    was used as it was passed (contiguous, plain storage) and the native
+    module is there."""
+    if _lib.host() is None:
+        return
     keys = (_tensor_key(q), _tensor_key(lens), _new_key(new[0]), _new_key(new[1]))
     if not all(k is None or k[-1] for k in keys):  # the caches: prepare() looks
         return
