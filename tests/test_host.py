@@ -458,29 +458,39 @@ def test_timing_replicas_and_warmup_floor():
     assert warmup_replays_needed(20, 0, 2.0, 0.5) == 1
 
 
-def test_prepared_call_key_tracks_what_the_argument_block_depends_on():
-    """The workspace's checked argument block is reused only under an equal
-    key: a tensor's key changes with its storage address, shape, dtype and
-    layout -- also when the same tensor object is resized or restrided in
-    place -- and a workspace without a prepared call, or with another key,
-    yields none."""
-    from tritonkv_amd.kernels.fused_decode_attn import _new_key, _prepared, _tensor_key
+def test_prepared_calls_run_only_for_the_form_that_was_checked():
+    """A kept call compares every tensor with the form that was checked and
+    launches nothing for another: a tensor read in place by storage address,
+    shape, dtype and layout -- also when the same tensor object is resized or
+    restrided in place -- and one that may move by shape, dtype and layout.  A
+    workspace without a prepared call, or with another key, yields none."""
+    from tritonkv_amd import _lib
+    from tritonkv_amd.kernels.fused_decode_attn import _OUT_OFFSET, _prepared
+
+    def prepare(*slots):
+        return _lib.host().prepare(bytes(_lib.DecodeArgs()), _lib.address("tkv_fused_decode_attention"),
+                                   0, slots, None)
+
+    def refused(call, *tensors):
+        return _lib.host().run(call, *tensors) is None
 
     t = torch.zeros(2, 3, 64, 16, dtype=torch.uint8)
-    k0 = _tensor_key(t)
-    assert _tensor_key(t) == k0
-    assert _tensor_key(torch.zeros_like(t)) != k0                 # another storage
+    moves = torch.zeros(2, 8)
+    call = prepare((t, -1, 1), (moves, _OUT_OFFSET, 1))
+    assert refused(call, torch.zeros_like(t), moves)                # another storage
+    assert refused(call, t.view(torch.int8), moves)                 # dtype view
+    assert refused(call, t.transpose(2, 3), moves)                  # layout
+    assert refused(call, None, moves) and refused(call, t, None) and refused(call, t)
+    assert refused(call, t, moves.half()) and refused(call, t, torch.zeros(8, 2))
+    assert refused(call, t, torch.zeros(2, 16)[:, ::2])
     t2 = torch.zeros(2, 3, 64, 16, dtype=torch.uint8)
-    ptr = t2.data_ptr()
-    t2.resize_(2, 3, 32, 16)                                      # same storage, new shape
-    assert t2.data_ptr() == ptr and _tensor_key(t2)[1] != k0[1]
-    v = t.view(torch.int8)
-    assert v.data_ptr() == t.data_ptr() and _tensor_key(v) != k0  # dtype view
-    tt = t.transpose(2, 3)
-    assert tt.data_ptr() == t.data_ptr() and _tensor_key(tt) != k0  # layout
-    assert _tensor_key(None) is None and _new_key(None) is None
-    assert _new_key(t) == _new_key(torch.ones_like(t))             # new rows may move
-    assert _new_key(t) != _new_key(t.half())
+    call, ptr = prepare((t2, -1, 1), (None, -1, 1)), t2.data_ptr()
+    t2.resize_(2, 3, 32, 16)                                        # same storage, new shape
+    assert t2.data_ptr() == ptr and refused(call, t2, None)
+    t2.resize_(2, 3, 64, 16)
+    assert refused(call, t2, moves)                                 # one that was not given
+    assert prepare((t.transpose(2, 3), -1, 1)) is None              # never kept
+    assert prepare((moves.view(-1)[1:], _OUT_OFFSET, 16)) is None   # misaligned
 
     class Prep:
         key = ("a", 1)

@@ -452,17 +452,6 @@ def new_token_args(k_new, v_new, B: int, HKV: int, D: int, device):
     return out[0], out[1], int(out[0].dtype == torch.float32)
 
 
-def _tensor_key(t):
-    """What the argument checks and the argument block depend on for a tensor
-    the call reads in place: its storage, shape, dtype and layout."""
-    return None if t is None else (t.data_ptr(), t.shape, t.dtype, t.is_contiguous())
-
-
-def _new_key(t):
-    """The same for the new token's rows, whose storage may change every step."""
-    return None if t is None else (t.shape, t.dtype, t.is_contiguous())
-
-
 class _PreparedCall:
     """A checked decode call, kept in the caller's ``_workspace`` under ``"call"``.
     ``key`` holds the options it was planned with; the forms of its tensors
@@ -499,12 +488,9 @@ _OUT_OFFSET, _Q_OFFSET, _K_NEW_OFFSET, _V_NEW_OFFSET = (
 def _keep_call(ws, key, args, entry, what, out, buffers, q, caches, lens, new=(None, None),
                window=None):
     """Put a call that just ran into the workspace for reuse, if every tensor
-    was used as it was passed (contiguous, plain storage) and the native
-    module is there."""
+    was used as it was passed (contiguous, plain storage: prepare() looks) and
+    the native module is there."""
     if _lib.host() is None:
-        return
-    keys = (_tensor_key(q), _tensor_key(lens), _new_key(new[0]), _new_key(new[1]))
-    if not all(k is None or k[-1] for k in keys):  # the caches: prepare() looks
         return
     slots = ((out, _OUT_OFFSET, 16), (q, _Q_OFFSET, 16), *((t, -1, 1) for t in caches),
              (lens, -1, 1), (new[0], _K_NEW_OFFSET, 1), (new[1], _V_NEW_OFFSET, 1))
