@@ -80,9 +80,11 @@ def _check_plan(B, S, kb, vb, G, lengths, plan, order):
     (50, 3000, 4, 2, 8, "ragged", (4, 1, False)),  # paired tiles, too short for an order
     (50, 8300, 2, 2, 4, "ragged", (12, 1, True)),
     (64, 20000, 2, 2, 4, "ragged", (4, 2, True)),  # four workgroups per CU
-    (16, 4097, 4, 4, 4, "ragged", (8, 2, False)),  # half a unit per CU
+    (16, 4000, 4, 4, 4, "ragged", (8, 2, False)),  # half a unit per CU
+    (16, 4097, 4, 4, 4, "ragged", (4, 4, False)),
+    (16, 12321, 4, 2, 8, "ragged", (4, 4, False)),
     (20, 9001, 4, 2, 8, "ragged", (4, 6, False)),  # below a unit per CU: cut finely
-    (32, 66000, 4, 2, 8, "ragged", (8, 2, True)),  # one unit per CU, long rows
+    (32, 66000, 4, 2, 8, "ragged", (4, 6, True)),  # one unit per CU, long rows cut finely
 ])
 def test_rules_match_the_oracle(B, S, kb, vb, G, lengths, plan):
     from tritonkv_amd.kernels import fused_decode_attention

@@ -156,21 +156,30 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
 
     ``fine``: the caller runs short ragged pieces in 4-wave workgroups
     (``choose_waves``), of which a CU holds two or three, so that a finer cut
-    costs little and evens out rows of different lengths.  Where the rules
-    above leave one split on half a unit to one unit per CU (or two, at exactly
-    half), a long enough history is cut into 4 workgroups per CU, in pieces
-    of at least 1024 tokens.  The fuller the grid, the longer the rows must be
-    for that to pay (HKV = 8, lengths from S/16 or S/64 to S, mean of three draws,
-    as above -> cut, us, for 4-bit G = 4 / 2-bit G = 4 / K4V2 G = 8):
+    costs little and evens out rows of different lengths.  HKV = 8; as above ->
+    cut, us, mean of three draws of lengths from S/16 or S/64 to S (eight draws from
+    half a unit and from one unit on), for 4-bit G = 4 / 2-bit G = 4 / K4V2 G = 8:
 
-    * 17 rows of up to 4096: 20.5 -> 17.1, 18.8 -> 15.8, 21.0 -> 17.8;
-    * 24 rows: 4096 21.4 -> 22.3, 19.2 -> 19.4, 21.2 -> 21.7 (not cut); 8192
-      35.2 -> 31.6, 29.9 -> 25.1, 33.2 -> 29.0;
-    * 28 rows: 8192 38.8 -> 43.4, 31.3 -> 30.1, 35.7 -> 41.3 (not cut); 16384
-      65.3 -> 55.6, 53.8 -> 42.2, 59.9 -> 49.4;
-    * 16 rows: 8192 25.7 -> 26.1, 22.5 -> 22.2, 24.8 -> 25.9 and 16384 42.2 ->
-      44.4, 35.1 -> 31.0, 38.4 -> 41.9 (not cut); 32768 72.4 -> 65.1, 58.8 ->
-      46.1, 65.2 -> 59.0.
+    * more than half a unit to one unit per CU, where the rules above leave one
+      split: 4 workgroups per CU in pieces of at least 1024 tokens.  The fuller
+      the grid, the longer the rows must be for that to pay.  17 rows of up to
+      4096: 20.5 -> 17.1, 18.8 -> 15.8, 21.0 -> 17.8; 24 rows: 4096 21.4 -> 22.3, 19.2 ->
+      19.4, 21.2 -> 21.7 (not cut), 8192 35.2 -> 31.6, 29.9 -> 25.1, 33.2 -> 29.0; 28
+      rows: 8192 38.8 -> 43.4, 31.3 -> 30.1, 35.7 -> 41.3 (not cut), 16384 65.3 -> 55.6,
+      53.8 -> 42.2, 59.9 -> 49.4;
+    * half a unit per CU, in two splits above: the same in pieces of 1024 tokens up
+      to 8192, of 4096 beyond.  16 rows of up to 8192: 25.4 -> 25.9, 22.0 -> 21.9, 24.1 ->
+      25.8, in page pools 27.2 -> 26.7, 24.7 -> 23.5, 27.2 -> 27.0 (groups of 128 28.9 ->
+      25.8); 16384: 40.4 -> 38.1, 33.7 -> 31.3, 37.4 -> 33.9 (in pieces of 1024-2048 41.4,
+      30.1, 39.6), paged 43.6 -> 39.3, 39.4 -> 35.4, 43.2 -> 38.2; 32768: 73.5 -> 69.3,
+      57.7 -> 48.2, 64.8 -> 63.0, paged 78.3 -> 71.5, 68.9 -> 56.4, 75.2 -> 65.4;
+    * one to two units per CU and 65536 tokens or more: pieces of 8192-16384
+      tokens.  32 rows of up to 65536: 225.1 -> 221.7, 156.3 -> 151.5, 191.1 -> 188.7,
+      paged 228.6 -> 226.3, 171.7 -> 165.3, 202.9 -> 199.4; 48 rows: 339.8 -> 333.7, 232.9 ->
+      217.3, 284.8 -> 284.4; 40 rows of up to 98304: 398.7 -> 392.0, 272.2 -> 256.7, 339.4 ->
+      336.6 (single draws lie within 7% of that either way); head dim 64, one draw,
+      150 -> 126.  At 49152 it is even (181.9 -> 181.1, 127.8 -> 127.7, 157 -> 154, groups of
+      128 157 -> 163).
 
     Returned in units of ``block_n`` blocks so the reference's tightening
     applies unchanged.
@@ -182,14 +191,13 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
     if units >= cu:
         if not ragged or S < 16384:
             return 1
-        return min(max(2, S // 32768), _cdiv(S, block_n))
+        piece = 32768 if units >= 2 * cu or S < 65536 or not fine else 10922
+        return min(max(2, S // piece), _cdiv(S, block_n))
     if ragged and fine and 2 * units >= cu:
-        if 2 * units == cu:
-            least = 32768
-        else:
-            least = 4096 if 8 * units <= 5 * cu else 8192 if 4 * units <= 3 * cu else 16384
+        least = 4096 if 8 * units <= 5 * cu else 8192 if 4 * units <= 3 * cu else 16384
+        pieces = _cdiv(S, 4096) if 2 * units == cu and S > 8192 else S // 1024
         if S >= least:
-            return max(1, min(4 * cu // units, S // 1024, _cdiv(S, block_n)))
+            return max(1, min(4 * cu // units, pieces, _cdiv(S, block_n)))
     workgroups = min(cu, max(32, units * S // tokens_per_workgroup))
     want = max(1, workgroups // units)
     max_splits = max(1, S // max(tokens_per_workgroup // 4, block_n))
