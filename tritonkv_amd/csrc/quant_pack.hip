@@ -352,7 +352,7 @@ quantize_tokens_kernel(TokenSource src, int HKV, int N, int tiles,
 // 16 / P of the dwords, and two exchanges with neighbouring lanes turn them into
 // 8-byte pieces of packed rows.
 // Bound by HBM: 4 x 8 heads of 8192 tokens, D = 128, fp16 to 2-bit, from a
-// token-major source: 18.1 us (4.5 TB/s); byte columns per lane (2-byte loads,
+// token-major source: 18.1 us (4.4 TB/s); byte columns per lane (2-byte loads,
 // byte stores) took 35.9 us after a 36.4 us copy to contiguous keys.
 template <int D, int NB, bool F32>
 struct KeyBlock {
