@@ -65,7 +65,7 @@ def _check_plan(B, S, kb, vb, G, lengths, plan, order):
     if fda.compute_units() != 256:
         return
     ragged = lengths == "ragged"
-    _, ns, split = fda.plan_splits(S, 64, None, B, 8, G, ragged=ragged)
+    _, ns, split = fda.plan_splits(S, 64, None, B, 8, G, ragged=ragged, fine=True)
     waves = fda.choose_waves(B, 8, G, split, ns, k_nbits=kb, v_nbits=vb, group_size=32, ragged=ragged)
     assert (waves, ns, order) == plan
 

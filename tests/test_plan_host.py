@@ -22,10 +22,20 @@ def _cus(monkeypatch):
 def test_ragged_batches_are_cut_where_that_was_measured_to_pay(B, S, splits):
     from tritonkv_amd.kernels.fused_decode_attn import plan_splits
 
-    assert plan_splits(S, 64, None, B, 8, 4, ragged=True)[1] == splits
-    # the fp16 control and per-channel keys keep the even cut
-    even = plan_splits(S, 64, None, B, 8, 4, ragged=True, fine=False)[1]
+    assert plan_splits(S, 64, None, B, 8, 4, ragged=True, fine=True)[1] == splits
+    # the fp16 control, per-channel keys and callers with partials of their own keep the even cut
+    even = plan_splits(S, 64, None, B, 8, 4, ragged=True)[1]
     assert even == ({16: 2}.get(B, 1) if B < 32 else max(2, S // 32768))
+
+
+def test_the_plan_of_other_callers_fits_the_static_scratch():
+    """48 rows of 64 query heads and up to 131072 tokens: the partials of the plan
+    a caller without a workspace makes (tkv_fused_decode_attention_noalloc)."""
+    from tritonkv_amd import _lib
+    from tritonkv_amd.kernels import plan_splits
+
+    _, ns, _ = plan_splits(131072, 64, None, 48, 8, 8, ragged=True)
+    assert ns == 4 and 48 * 64 * ns * (128 + 2) * 4 <= _lib.NOALLOC_SCRATCH_BYTES
 
 
 FP16, K4, K2, K42 = (16, 16, 0), (4, 4, 32), (2, 2, 32), (4, 2, 32)

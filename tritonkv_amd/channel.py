@@ -187,8 +187,7 @@ def channel_decode_attention(
     group = HQ // HKV
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     ragged = q_lens is not None and not equal_lengths
-    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged,
-                                            fine=False)
+    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged)
     q_in = q
     if q.dtype not in (torch.float16, torch.float32):
         q = q.float()

@@ -86,7 +86,7 @@ def fp16_decode_attention(
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     ragged = seq_lens is not None and not equal_lengths
     _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group,
-                                            TOKENS_PER_WORKGROUP_FP16, ragged=ragged, fine=False)
+                                            TOKENS_PER_WORKGROUP_FP16, ragged=ragged)
 
     q_in = q
     if q.dtype not in (torch.float16, torch.float32):

@@ -118,7 +118,7 @@ MAX_SPLITS = 65535  # grid y-dimension limit
 
 def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
                        tokens_per_workgroup: int = TOKENS_PER_WORKGROUP, *,
-                       ragged: bool = False, fine: bool = True) -> int:
+                       ragged: bool = False, fine: bool = False) -> int:
     """Split count used when the caller passes ``num_splits=None``.
 
     Chosen from sweeps on MI355X (split count x workgroup size, DRAM-resident
@@ -154,11 +154,13 @@ def default_num_splits(B: int, HKV: int, G: int, S: int, block_n: int,
     unsplit.  Equal lengths pay for the second split (Llama-3-8B shape:
     206.6 vs 200.7 us).
 
-    ``fine``: the caller runs short ragged pieces in 4-wave workgroups
-    (``choose_waves``), of which a CU holds two or three, so that a finer cut
-    costs little and evens out rows of different lengths.  HKV = 8; as above ->
-    cut, us, mean of three draws of lengths from S/16 or S/64 to S (eight draws from
-    half a unit and from one unit on), for 4-bit G = 4 / 2-bit G = 4 / K4V2 G = 8:
+    ``fine`` (the quantized entry points; off for other callers of this plan, whose
+    partials may be sized for the splits above): the caller runs short ragged
+    pieces in 4-wave workgroups (``choose_waves``), of which a CU holds two or
+    three, so that a finer cut costs little and evens out rows of different
+    lengths.  HKV = 8; as above -> cut, us, mean of three draws of lengths from S/16
+    or S/64 to S (eight draws from half a unit and from one unit on), for 4-bit G = 4 /
+    2-bit G = 4 / K4V2 G = 8:
 
     * more than half a unit to one unit per CU, where the rules above leave one
       split: 4 workgroups per CU in pieces of at least 1024 tokens.  The fuller
@@ -297,7 +299,7 @@ def choose_waves(B: int, HKV: int, G: int, split_size: int, num_splits: int = 0,
 
 def plan_splits(S: int, block_n: int, num_splits: int | None, B: int, HKV: int, G: int,
                 tokens_per_workgroup: int = TOKENS_PER_WORKGROUP, *, ragged: bool = False,
-                fine: bool = True):
+                fine: bool = False):
     """Reference split arithmetic (:486-499) -> (block_n, num_splits, split_size).
 
     One addition: the count is capped at 65535 before tightening (splits are
@@ -596,7 +598,8 @@ def fused_decode_attention(
     group = HQ // HKV
     sm_scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     ragged = seq_lens is not None and not equal_lengths
-    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged)
+    _, num_splits, split_size = plan_splits(S, block_n, num_splits, B, HKV, group, ragged=ragged,
+                                            fine=True)
 
     q_in = q
     if q.dtype not in (torch.float16, torch.float32):
