@@ -1,10 +1,12 @@
 """Decode over caches whose blocks start inside a cache line (S no multiple of 32).
 
-Splits of 4096 tokens or more then count their chunks from a multiple of 32
-rows of the tensor and mask the rows before the split: the chunk before the
-block's start (read as zeros), before a later split's start (the previous
-split's rows), and a first chunk that is also the last, with and without the
-appended token in it.  Against the oracle's fp32 attention over the same codes.
+Splits of 4096 tokens or more of the long-split forms (paired tiles, which small
+grids run from 8192 tokens, and one tile at a time above 8 query heads) then count
+their chunks from a multiple of 32 rows of the tensor and mask the rows before the
+split: the chunk before the block's start (read as zeros), before a later split's
+start (the previous split's rows), and a first chunk that is also the last, with
+and without the appended token in it.  Against the oracle's fp32 attention over
+the same codes.
 """
 
 from __future__ import annotations
@@ -18,14 +20,14 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 CASES = [  # nbits, gs, HQ, HKV, D, S, num_splits
-    (4, 32, 8, 2, 128, 4127, 1),     # one tile at a time
-    (4, 32, 8, 2, 128, 8250, 2),     # a second split that starts at a block of 64
+    (4, 32, 8, 2, 128, 4127, 1),     # one tile at a time: not aligned
+    (4, 32, 8, 2, 128, 8250, 2),     # ... and a second split that starts at a block of 64
     (4, 32, 12, 2, 128, 8251, 1),    # paired tiles
     (2, 32, 8, 2, 128, 8263, 1),     # 12 waves
-    (2, 128, 8, 2, 128, 8250, 1),    # one group per row, pairs of metadata
-    (2, 128, 8, 2, 128, 8251, 1),    # ... odd S: not aligned
+    (2, 128, 8, 2, 128, 8250, 1),    # one group per row: not aligned
+    (2, 128, 8, 2, 128, 8251, 1),    # ... odd S
     (4, 16, 32, 2, 128, 4099, 1),    # 16 head columns
-    (2, 64, 4, 2, 64, 8199, 1),
+    (2, 64, 4, 2, 64, 8199, 1),      # one group per row
 ]
 
 
@@ -42,7 +44,8 @@ def test_unaligned_blocks_match_the_oracle(case):
 @pytest.mark.parametrize("nbits,HQ,S", [(4, 8, 4127), (2, 8, 8263), (4, 12, 8251)])
 @pytest.mark.parametrize("append", [False, True])
 def test_short_rows_of_unaligned_blocks(nbits, HQ, S, append):
-    """Rows that end in the first chunk, just past it, and at the capacity."""
+    """Rows that end in the first chunk, just past it, and at the capacity (4-bit at
+    4127 not aligned)."""
     from tritonkv_amd.kernels import fused_decode_attention
     from tritonkv_amd.quantize import append_kv
 
