@@ -28,6 +28,9 @@ CASES = [  # nbits, gs, HQ, HKV, D, S, num_splits
     (2, 128, 8, 2, 128, 8251, 1),    # ... odd S
     (4, 16, 32, 2, 128, 4099, 1),    # 16 head columns
     (2, 64, 4, 2, 64, 8199, 1),      # one group per row
+    (4, 32, 8, 2, 128, 16451, 2),    # paired tiles, a second split
+    (2, 32, 8, 2, 128, 16469, 2),    # ... in 12 waves
+    (4, 16, 32, 2, 128, 8251, 2),    # 16 head columns, a second split
 ]
 
 
